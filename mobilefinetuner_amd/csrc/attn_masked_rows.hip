@@ -65,32 +65,121 @@ __device__ __forceinline__ float wave_sum(float x) {
 
 template <typename T> __device__ __forceinline__ float ld(const T* p) { return (float)*p; }
 
+// VEC consecutive elements of a row (one 16-byte access, or a single one).
+template <typename T, int VEC> struct alignas(VEC * sizeof(T)) Pack {
+    T x[VEC];
+};
+
+constexpr int kFwdThreads = 1024;
+
+// Lanes that span a row of D elements, VEC to a lane: a power of two, so that
+// the rows a workgroup holds at once divide its threads.
+__host__ __device__ constexpr int row_lanes(int D, int VEC) {
+    int n = 1;
+    while (n * VEC < D) n *= 2;
+    return n;
+}
+
+// The forward's share of a row: one 128-byte line per workgroup where rows
+// are read in vectors, so that many groups of lanes share the rows.
+__host__ __device__ constexpr int fwd_lanes(int D, int VEC) {
+    const int n = row_lanes(D, VEC), most = VEC > 1 ? 8 : 64;
+    return n < most ? n : most;
+}
+
 // Forward: O_i = mean of V over T_i for every masked row, all query heads of
-// the kv head.  Workgroup = (64-row chunk, batch x kv head); thread = column.
-// The sum over [0, len) is formed once per workgroup, the window part is
-// rolled along the rows; both in double.
-template <typename T>
-__global__ __launch_bounds__(256) void attn_fwd_masked_rows(MaskedArgs a) {
-    const int S = a.S, D = a.D, d = threadIdx.x;
+// the kv head.  Bound by the latency of reading [0, len) and the window.
+// Workgroup = (G rows, batch x kv head, a line's columns), G = 1024 /
+// fwd_lanes (128 rows of 64 bf16 columns): group g of fwd_lanes threads sums
+// every G-th row of T_r0 (r0 the workgroup's first masked row), eight rows'
+// loads in flight, the groups' sums are added through LDS, and group g then
+// owns row r0 + g, whose T differs from T_r0 by one entering and one leaving
+// row per step: a prefix sum over the groups.  All sums in double.  One thread
+// per column walking the rows alone took 245 us at B 3, Hkv 1, S 1000, D 256,
+// window 512 with lengths down to 390; whole rows to a workgroup 16; this 10.
+template <typename T, int VEC>
+__global__ __launch_bounds__(kFwdThreads) void attn_fwd_masked_rows(MaskedArgs a) {
+    typedef Pack<T, VEC> P;
+    __shared__ double part[VEC][kFwdThreads], seg[kFwdThreads];
+    const int S = a.S, D = a.D, tid = threadIdx.x;
+    const int lanes = fwd_lanes(D, VEC), G = kFwdThreads / lanes, g = tid / lanes;
+    const int d = ((int)blockIdx.z * lanes + tid % lanes) * VEC;
     const int bk = blockIdx.y, b = bk / a.Hkv, hk = bk % a.Hkv;
     const MaskedRows mr = masked_rows(a, b);
-    const int r0 = max((int)blockIdx.x * 64, mr.first()), r1 = min((int)blockIdx.x * 64 + 64, S);
-    if (r0 >= r1 || d >= D) return;
-    const T* V = (const T*)a.v + a.sv.at(b, hk) + d;
+    const int r0 = max((int)blockIdx.x * G, mr.first()), r1 = min((int)blockIdx.x * G + G, S);
+    if (r0 >= r1) return;
+    const bool live = d < D;  // D is a multiple of VEC
+    const T* V = (const T*)a.v + a.sv.at(b, hk) + (live ? d : 0);
     const int64_t lv = a.sv.s;
-    double pre = 0.0;
-    for (int j = 0; j < mr.len; ++j) pre += ld(V + (int64_t)j * lv);
-    int lo = mr.tlo(r0), hi = mr.thi(r0);
-    double win = 0.0;
-    for (int j = lo; j <= hi; ++j) win += ld(V + (int64_t)j * lv);
-    for (int i = r0; i < r1; ++i) {
-        const int nlo = mr.tlo(i), nhi = mr.thi(i);
-        for (; hi < nhi; ++hi) win += ld(V + (int64_t)(hi + 1) * lv);
-        for (; lo < nlo; ++lo) win -= ld(V + (int64_t)lo * lv);
-        const float o = (float)((pre + win) / (double)mr.count(i));
-        for (int h = hk * a.group; h < (hk + 1) * a.group; ++h)
-            ((T*)a.o)[a.so.at(b, h) + (int64_t)i * a.so.s + d] = (T)o;
+    double acc[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) acc[e] = 0.0;
+    // T_r0 as one list: [0, len), then [lo, hi].
+    const int lo = mr.tlo(r0), total = mr.count(r0);
+    constexpr int U = 8;
+    for (int n0 = g; n0 < total; n0 += U * G) {
+        P x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int n = min(n0 + u * G, total - 1);
+            x[u] = *reinterpret_cast<const P*>(V + (int64_t)(n < mr.len ? n : lo + n - mr.len) * lv);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (n0 + u * G < total)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) acc[e] += (double)(float)x[u].x[e];
     }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) part[e][tid] = acc[e];
+    __syncthreads();
+    // A column's G values are handled by Q = G / VEC threads, VEC values each:
+    // thread (q, element ce, lane cl).
+    const int cols = lanes * VEC, q = tid / cols, ce = (tid % cols) / lanes, cl = tid % lanes;
+    const int Q = kFwdThreads / cols;
+    double* mine = &part[ce][q * VEC * lanes + cl];  // values s * lanes apart
+    double sum = 0.0;
+#pragma unroll
+    for (int s = 0; s < VEC; ++s) sum += mine[s * lanes];
+    seg[tid] = sum;
+    __syncthreads();
+    sum = 0.0;  // over T_r0
+    for (int s = 0; s < Q; ++s) sum += seg[s * cols + tid % cols];
+    // Row i = r0 + g: what entered T since row i - 1 less what left it.
+    const int i = r0 + g;
+    const bool in = i < r1;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) acc[e] = 0.0;
+    if (in && g > 0) {
+        const P add = *reinterpret_cast<const P*>(V + (int64_t)mr.thi(i) * lv);
+        const P sub = *reinterpret_cast<const P*>(V + (int64_t)mr.tlo(i - 1) * lv);
+        const bool enters = mr.thi(i) > mr.thi(i - 1), leaves = mr.tlo(i) > mr.tlo(i - 1);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+            acc[e] = (enters ? (double)(float)add.x[e] : 0.0) - (leaves ? (double)(float)sub.x[e] : 0.0);
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) part[e][tid] = acc[e];
+    __syncthreads();
+    double d_seg = 0.0;
+#pragma unroll
+    for (int s = 0; s < VEC; ++s) d_seg += mine[s * lanes];
+    seg[tid] = d_seg;
+    __syncthreads();
+    for (int s = 0; s < q; ++s) sum += seg[s * cols + tid % cols];
+#pragma unroll
+    for (int s = 0; s < VEC; ++s) {
+        sum += mine[s * lanes];
+        mine[s * lanes] = sum;
+    }
+    __syncthreads();
+    if (!in || !live) return;
+    const double n = (double)mr.count(i);
+    P o;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o.x[e] = (T)(float)(part[e][tid] / n);
+    for (int h = hk * a.group; h < (hk + 1) * a.group; ++h)
+        *reinterpret_cast<P*>((T*)a.o + a.so.at(b, h) + (int64_t)i * a.so.s + d) = o;
 }
 
 // This lane's columns lane + 64 c (c < 4, D <= 256) of a row.
@@ -110,13 +199,60 @@ __device__ __forceinline__ float dot4(const float (&x)[4], const float (&y)[4]) 
 template <typename T>
 __device__ void masked_dq_row(const MaskedArgs& a, const MaskedRows& mr, int b, int h, int i);
 
-template <typename T>
+// Bit i of the result: row r0 + i of dO (n <= 16 rows) holds a non-zero.  The
+// rows' loads are in flight together (one row after the other, 16 memory
+// round trips per wave, took 40 us at the shape above; now 5).
+template <typename T, int VEC>
+__device__ __forceinline__ unsigned nonzero_rows(const T* dO, int64_t ld, int D, int n) {
+    typedef Pack<T, VEC> P;
+    const int lane = threadIdx.x & 63;
+    unsigned m = 0;
+    if constexpr (VEC > 1) {
+        const int lanes = row_lanes(D, VEC), rpw = 64 / lanes, q = lane / lanes, d = (lane % lanes) * VEC;
+        const unsigned long long row = lanes == 64 ? ~0ull : (1ull << lanes) - 1;
+        const T* p = dO + (d < D ? d : 0);
+        for (int r0 = 0; r0 < n; r0 += 8 * rpw) {
+            P x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = *reinterpret_cast<const P*>(p + (int64_t)min(r0 + u * rpw + q, n - 1) * ld);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                bool nz = false;
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) nz |= (float)x[u].x[e] != 0.f;
+                const unsigned long long hit = __ballot(nz && d < D);
+                if (!hit) continue;
+                for (int r = 0; r < rpw && r0 + u * rpw + r < n; ++r)
+                    if (hit >> (r * lanes) & row) m |= 1u << (r0 + u * rpw + r);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            bool nz = false;
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                nz |= u < n && lane + 64 * c < D && (float)dO[(int64_t)min(u, n - 1) * ld + min(lane + 64 * c, D - 1)] != 0.f;
+            if (__any(nz)) m |= 1u << u;
+        }
+    }
+    return m;
+}
+
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void attn_bwd_masked_dq(MaskedArgs a) {
     const int bh = blockIdx.y, b = bh / a.Hq, h = bh % a.Hq;
     const MaskedRows mr = masked_rows(a, b);
     const int r0 = max((int)blockIdx.x * 64 + 16 * (int)(threadIdx.x >> 6), mr.first());
     const int r1 = min((int)blockIdx.x * 64 + 16 * (int)(threadIdx.x >> 6) + 16, a.S);
-    for (int i = r0; i < r1; ++i) masked_dq_row<T>(a, mr, b, h, i);
+    if (r0 >= r1) return;
+    const unsigned active =
+        nonzero_rows<T, VEC>((const T*)a.dO + a.sdo.at(b, h) + (int64_t)r0 * a.sdo.s, a.sdo.s, a.D, r1 - r0);
+    const int lane = threadIdx.x & 63;
+    if (lane < r1 - r0) a.row_active[((int64_t)b * a.Hq + h) * a.S + r0 + lane] = active >> lane & 1;
+    // a row whose dO is zero has dq_i = 0, as the main pass left it
+    for (int i = r0; i < r1; ++i)
+        if (active >> (i - r0) & 1) masked_dq_row<T>(a, mr, b, h, i);
 }
 
 template <typename T>
@@ -126,13 +262,8 @@ __device__ void masked_dq_row(const MaskedArgs& a, const MaskedRows& mr, int b, 
     float g[4], o[4];
     load_row4((const T*)a.dO + a.sdo.at(b, h) + (int64_t)i * a.sdo.s, D, g);
     load_row4((const T*)a.o + a.so.at(b, h) + (int64_t)i * a.so.s, D, o);
-    const bool nz = __any(g[0] != 0.f || g[1] != 0.f || g[2] != 0.f || g[3] != 0.f);
     const float dl = wave_sum(dot4(g, o));
-    if (lane == 0) {
-        a.row_active[ri] = nz ? 1 : 0;
-        a.row_delta[ri] = dl;
-    }
-    if (!nz) return;  // dq_i = 0, as the main pass left it
+    if (lane == 0) a.row_delta[ri] = dl;
     const T* K = (const T*)a.k + a.sk.at(b, hk);
     const T* V = (const T*)a.v + a.sv.at(b, hk);
     const float inv_c = 1.f / (float)mr.count(i);
@@ -166,6 +297,16 @@ __global__ __launch_bounds__(256) void attn_bwd_masked_dkdv(MaskedArgs a) {
     const int bk = blockIdx.y, b = bk / a.Hkv, hk = bk % a.Hkv;
     const MaskedRows mr = masked_rows(a, b);
     if (mr.first() >= a.S) return;
+    // No active row among the group's heads (their padded positions carry no
+    // loss): nothing to add.  Found by all threads together; each wave looking
+    // through the rows for each of its keys took 48 us at the shape above.
+    bool any = false;
+    for (int h = hk * a.group; h < (hk + 1) * a.group; ++h) {
+        const int* act = a.row_active + ((int64_t)b * a.Hq + h) * a.S;
+#pragma unroll 4
+        for (int i = mr.first() + (int)threadIdx.x; i < a.S; i += 256) any |= act[i] != 0;
+    }
+    if (!__syncthreads_or(any)) return;
     const int j0 = (int)blockIdx.x * 64 + 16 * (int)(threadIdx.x >> 6);
     for (int j = j0; j < min(j0 + 16, a.S); ++j) masked_dkdv_key<T>(a, mr, b, hk, j);
 }
@@ -240,6 +381,14 @@ MaskedArgs masked_args(const AttnShape& s) {
     return a;
 }
 
+// Elements per access of a row: 16 bytes where every row starts on 16 bytes.
+// Strides the caller gives are multiples of 16 bytes (checked by the C ABI);
+// contiguous rows are when D is.
+int row_vec(const AttnShape& s) {
+    const int w = s.bf16 ? 8 : 4;
+    return s.D % w == 0 ? w : 1;
+}
+
 }  // namespace
 
 size_t masked_rows_workspace_bytes(const AttnShape& s) {
@@ -253,11 +402,21 @@ hipError_t launch_fwd_masked_rows(const AttnShape& s, const void* v, void* o, hi
     MaskedArgs a = masked_args(s);
     a.v = v;
     a.o = o;
-    const dim3 grid((unsigned)((s.S + 63) / 64), (unsigned)(s.B * s.Hkv));
-    if (s.bf16)
-        hipLaunchKernelGGL(attn_fwd_masked_rows<bf16>, grid, dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL(attn_fwd_masked_rows<float>, grid, dim3(256), 0, st, a);
+    const int vec = row_vec(s), lanes = fwd_lanes(a.D, vec), rows = kFwdThreads / lanes;
+    const dim3 grid((unsigned)((s.S + rows - 1) / rows), (unsigned)(s.B * s.Hkv),
+                    (unsigned)((a.D + lanes * vec - 1) / (lanes * vec)));
+    const dim3 blk(kFwdThreads);
+    if (s.bf16) {
+        if (vec > 1)
+            hipLaunchKernelGGL((attn_fwd_masked_rows<bf16, 8>), grid, blk, 0, st, a);
+        else
+            hipLaunchKernelGGL((attn_fwd_masked_rows<bf16, 1>), grid, blk, 0, st, a);
+    } else {
+        if (vec > 1)
+            hipLaunchKernelGGL((attn_fwd_masked_rows<float, 4>), grid, blk, 0, st, a);
+        else
+            hipLaunchKernelGGL((attn_fwd_masked_rows<float, 1>), grid, blk, 0, st, a);
+    }
     return hipGetLastError();
 }
 
@@ -278,11 +437,18 @@ hipError_t launch_bwd_masked_rows(const AttnShape& s, const void* q, const void*
     a.row_active = reinterpret_cast<int*>(static_cast<char*>(scratch) + half);
     const dim3 gq((unsigned)((s.S + 63) / 64), (unsigned)(s.B * s.Hq));
     const dim3 gk((unsigned)((s.S + 63) / 64), (unsigned)(s.B * s.Hkv));
+    const bool vec = row_vec(s) > 1;
     if (s.bf16) {
-        hipLaunchKernelGGL(attn_bwd_masked_dq<bf16>, gq, dim3(256), 0, st, a);
+        if (vec)
+            hipLaunchKernelGGL((attn_bwd_masked_dq<bf16, 8>), gq, dim3(256), 0, st, a);
+        else
+            hipLaunchKernelGGL((attn_bwd_masked_dq<bf16, 1>), gq, dim3(256), 0, st, a);
         hipLaunchKernelGGL(attn_bwd_masked_dkdv<bf16>, gk, dim3(256), 0, st, a);
     } else {
-        hipLaunchKernelGGL(attn_bwd_masked_dq<float>, gq, dim3(256), 0, st, a);
+        if (vec)
+            hipLaunchKernelGGL((attn_bwd_masked_dq<float, 4>), gq, dim3(256), 0, st, a);
+        else
+            hipLaunchKernelGGL((attn_bwd_masked_dq<float, 1>), gq, dim3(256), 0, st, a);
         hipLaunchKernelGGL(attn_bwd_masked_dkdv<float>, gk, dim3(256), 0, st, a);
     }
     return hipGetLastError();

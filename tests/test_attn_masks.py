@@ -151,3 +151,16 @@ def test_window_forward_launch_shapes_agree(orc, dev):
         torch.cuda.synchronize()
         assert orc.max_rel(o.float().cpu().numpy(), ref["o"]) <= TOL["bf16"], balanced
         assert np.max(np.abs(lse.cpu().numpy() - ref["lse"])) <= 1e-3, balanced
+
+
+@pytest.mark.parametrize("case", [
+    (2, 2, 1, 300, 36, "bf16", True, 20, [0, 111]),   # rows not of whole 16-byte vectors
+    (1, 2, 2, 150, 6, "f32", True, 7, [33]),
+    (1, 2, 1, 67, 250, "f32", True, 5, [1]),          # four rows to a workgroup, one left over
+    (2, 4, 1, 333, 64, "bf16", True, 40, [50, 0]),    # 128 rows to a workgroup, the last partly filled
+    (2, 2, 2, 129, 256, "bf16", False, 0, [0, 3]),    # not causal: every row of a batch takes one mean
+], ids=_id)
+def test_rows_without_keys_match_oracle(orc, dev, case):
+    """Rows that see no key, at the edges of the row groups and vectors that
+    the masked-row kernels take, with gradients on those rows."""
+    test_masked_fwd_bwd_matches_oracle(orc, dev, case)
