@@ -262,3 +262,43 @@ def test_autograd_node(orc, dev):
     ref = orc.selected_ce(h.detach().cpu().numpy(), w.detach().cpu().numpy(), y.cpu().numpy(), -100, "mean", 2.0)
     assert _rel(orc, h.grad.cpu().numpy(), ref["grad_hidden"]) <= 1e-4
     assert _rel(orc, w.grad.cpu().numpy(), ref["grad_weight"]) <= 1e-4
+
+
+@pytest.mark.parametrize("case", [
+    (1, 9, 16385, "f32", "mean", 0),     # wide rows, one element past a whole pass, every start offset
+    (1, 10, 32771, "bf16", "sum", 1),    # the base one element off a 16-byte boundary
+    (1, 6, 16383, "f32", "none", 2),     # the widest of the 256-thread rows
+    (2, 5, 3, "f32", "mean", 1),         # rows shorter than a vector
+    (1, 700, 50257, "f32", "mean", 0),   # a gradient past the streaming-store size
+], ids=lambda c: "B{}S{}V{}-{}-{}-off{}".format(*c))
+def test_dense_unaligned_rows(dev, case):
+    """Rows that start off the vectors' boundaries, against double precision;
+    1e-5 relative for fp32 sums of up to 50257 terms, gradients to 2e-6 of
+    the largest (one exponential and one product in fp32)."""
+    import torch
+    from mobilefinetuner_amd import lm_loss as L
+    B, S, V, dtype, red, off = case
+    print(f"[case] dense unaligned {case}", flush=True)
+    g = torch.Generator(device=dev)
+    g.manual_seed(V + off)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    flat = (2.0 * torch.randn(off + B * S * V, device=dev, generator=g)).to(dt)
+    z = flat[off:].view(B, S, V)
+    y = torch.randint(0, V, (B, S), device=dev, generator=g, dtype=torch.int32)
+    y[0, 2] = -100
+    loss, lse = L.lm_cross_entropy(z, y, -100, red)
+    outer = torch.full(loss.shape, 0.5, device=dev)
+    grad = L.lm_cross_entropy_backward(z, y, lse, outer, -100, red)
+    z64, t = z.double().view(B * S, V), torch.full((B, S), -100, dtype=torch.int64, device=dev)
+    t[:, :-1] = y[:, 1:]
+    t = t.view(-1)
+    on = t >= 0
+    ref_lse = torch.logsumexp(z64, 1)
+    nll = torch.where(on, ref_lse - z64.gather(1, t.clamp(min=0)[:, None])[:, 0], 0.0)
+    ref = {"mean": nll.sum() / on.sum(), "sum": nll.sum(), "none": nll.view(B, S)}[red]
+    p = (z64 - ref_lse[:, None]).exp()
+    p[torch.arange(B * S, device=dev), t.clamp(min=0)] -= 1.0
+    rg = 0.5 * p * on[:, None] / (on.sum() if red == "mean" else 1)
+    assert torch.allclose(loss.double().view(-1), ref.reshape(-1), rtol=1e-5, atol=0)
+    assert torch.allclose(lse.double().view(-1), torch.where(on, ref_lse, 0.0), rtol=1e-5, atol=0)
+    assert float((grad.double().view(B * S, V) - rg).abs().max()) <= 2e-6 * float(rg.abs().max())
