@@ -22,9 +22,12 @@
  * and H a multiple of 64 the streaming forward is one fused kernel (the logits
  * GEMM with the online log-sum-exp in its epilogue; no logits are written),
  * and the backward's per-chunk G comes from the same kernel (logits
- * recomputed, G written in bf16).  The backward's two GEMMs per chunk, and the
- * logits GEMMs in the other cases, run on rocBLAS with a per-device handle
- * created on first use; the GEMM workspace comes from the caller's workspace.
+ * recomputed, G written in bf16).  With fp32 operands the three GEMMs of a
+ * chunk run on the bf16 matrix units, each operand as the exact sum of three
+ * bf16 numbers (csrc/gemm_f32.hip), with no more rounding than fp32 matrix
+ * instructions.  The bf16 backward's two GEMMs per chunk, and the logits GEMMs
+ * of the other bf16 shapes, run on rocBLAS with a per-device handle created on
+ * first use; the GEMM workspace comes from the caller's workspace.
  *
  * A label outside [0, V) that is not ignore_index makes the reference throw
  * ("lm_cross_entropy: label out of range").  A device cannot throw: the
@@ -48,7 +51,8 @@ typedef struct {
     int32_t dtype;         /* element type of logits (dense) or hidden and weight         */
     int32_t ignore_index;  /* skipped label value (reference default -100)                */
     int32_t reduction;     /* mft_reduction; streaming takes MEAN or SUM                  */
-    int32_t chunk;         /* streaming: vocabulary rows per GEMM chunk (0 = 16384)        */
+    int32_t chunk;         /* streaming: vocabulary rows per GEMM chunk (0 = 16384, or in
+                              fp32 as many as keep the chunk's logits within 128 MiB)     */
 } mft_lm_loss_desc;
 
 /* Workspace bytes of the forward and backward (dense or streaming per desc->H). */

@@ -356,7 +356,7 @@ template <int CPR> __host__ __device__ __forceinline__ constexpr int swz_tr16(in
 enum { SWZ_ROW = 0, SWZ_TR = 1, SWZ_DUAL = 2, SWZ_TR16 = 3 };
 
 // Scheduling-group masks of __builtin_amdgcn_sched_group_barrier.
-enum { SG_MFMA = 0x008, SG_DS_READ = 0x100 };
+enum { SG_VALU = 0x002, SG_MFMA = 0x008, SG_DS_READ = 0x100 };
 
 // Pin the order of an unrolled "operands read PF steps ahead" loop in the
 // current scheduling region.  A step reads R LDS operands and issues M

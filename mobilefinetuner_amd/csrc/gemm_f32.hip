@@ -1,0 +1,419 @@
+// fp32 matrix products from bf16 MFMAs.
+//
+// An fp32 number is the exact sum of three bf16 numbers: its top 8 significant
+// bits, the next 8 and the rest (split3, by truncation; both remainders are
+// exact in fp32).  With a = a1 + a2 + a3 and b likewise,
+//   a b = a1 b1 + a1 b2 + a2 b1 + a2 b2 + a1 b3 + a3 b1   (+ terms below 2^-22 a b)
+// and each product of two bf16 numbers is exact in the fp32 accumulator's
+// multiplier.  Six v_mfma_f32_32x32x16_bf16 then do the work of eight
+// v_mfma_f32_32x32x2_f32 in 6 x 32 instead of 8 x 64 cycles, and round the
+// accumulator 6 times per 16 values of k instead of 8.
+// What it gives (us, TFLOP/s of the fp32 product; rocBLAS's fp32 kernels beside
+// it): 512 x 16384 x 768 70 us, 183 (96 us); 512 x 768 x 16384 80 us, 161 (124
+// us, 880 without its split-k kernels); 2048 x 16384 x 1024 339 us, 203 (482
+// us), 1.2 PFLOP/s of bf16 products; 509 x 768 x 2304 23 us (21 us).  Error
+// against double precision 0.2 to 0.85 of the fp32 kernels'.  Bound by the
+// barrier per stage and the LDS traffic (72 KB per 128 x 128 x 16 stage)
+// beside the MFMAs.
+// Infinities: a remainder of inf, or 0 * inf among the six products, is NaN
+// where fp32 arithmetic may give inf; an element that comes out NaN is
+// computed again by a plain fp32 dot product (exact_dot).
+//
+// A workgroup (4 waves) owns a T x T tile of C and a range of BK-deep stages
+// of k (of every term in turn, so that a rank-r update is one or two more
+// stages).  A stage's fp32 values are loaded to registers two to three stages
+// ahead, split while the stage before is multiplied, and written to the other of two
+// LDS buffers ([plane][row][BK], 16-byte chunks XOR-swizzled): one barrier per
+// stage, with the split's VALU work between the MFMAs.  The waves read each
+// plane once: 12 KB of LDS reads per 24 MFMAs and wave at T = 128.  Either
+// operand may be stored with k contiguous (16-byte loads along k) or not
+// (loads along the rows, eight k per thread, which transposes in registers).
+#include "gemm_f32.h"
+
+#include <algorithm>
+
+#include "attn_common.h"
+#include "attn_geometry.h"
+#include "attn_kernels.h"
+
+namespace mft {
+namespace {
+
+constexpr int kPlanes = 3;
+
+struct Args {
+    GemmF32 g;
+    int tiles_m, tiles_n, slices, stages, per_slice;  // stages of all terms, and of one slice
+    int n0;     // stages of term 0
+    int whole;  // one slice and nothing to add to: written to C directly, else to partial
+};
+
+// E values as three planes of packed bf16.
+template <int E> struct Split {
+    uint32_t p[kPlanes][E / 2];
+};
+__device__ __forceinline__ uint32_t hi_pair(uint32_t lo, uint32_t hi) {
+    return __builtin_amdgcn_perm(hi, lo, 0x07060302u);  // (hi16 of lo, hi16 of hi)
+}
+template <int E> __device__ __forceinline__ Split<E> split3(const float* x) {
+    Split<E> s;
+#pragma unroll
+    for (int i = 0; i < E / 2; ++i) {
+        uint32_t a[2], b[2], c[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float v = x[2 * i + e];
+            a[e] = __float_as_uint(v);
+            const float r = v - __uint_as_float(a[e] & 0xffff0000u);
+            b[e] = __float_as_uint(r);
+            c[e] = __float_as_uint(r - __uint_as_float(b[e] & 0xffff0000u));
+        }
+        s.p[0][i] = hi_pair(a[0], a[1]);
+        s.p[1][i] = hi_pair(b[0], b[1]);
+        s.p[2][i] = hi_pair(c[0], c[1]);
+    }
+    return s;
+}
+
+// 16-byte chunk c (8 k) of row r in a plane of BK k per row.  Eight (BK = 16)
+// or four (32) rows fill the 64 banks, so the chunk turns with r / 8 or r / 4,
+// and 16 rows' reads of one chunk meet no bank twice.
+template <int BK> __device__ __forceinline__ int chunk_at(int r, int c) {
+    return BK == 16 ? r * 2 + (c ^ ((r >> 3) & 1)) : r * 4 + (c ^ ((r >> 2) & 3));
+}
+
+// One operand's stages on their way to LDS: each of the workgroup's NT threads
+// holds E = T * BK / NT consecutive k of one row.  k-contiguous storage (KC):
+// thread (row t / KG, k group t % KG); else (row t % T, k group t / T), a wave
+// reading 64 consecutive rows at each k.
+template <int T, int BK, int NT, bool KC> struct Loader {
+    static constexpr int E = T * BK / NT, KG = BK / E;
+    static_assert(E == 4 || E == 8, "one 16-byte load, or two");
+    int row, kg;
+    const float* base;  // this thread's first element of the fast path
+    int64_t step;       // elements from one stage to the next
+    bool fast;          // whole stages of the first term go by vector loads
+    __device__ __forceinline__ void init(const float* p, int64_t ld, int64_t r0, int64_t rows) {
+        row = KC ? (int)threadIdx.x / KG : (int)threadIdx.x % T;
+        kg = KC ? (int)threadIdx.x % KG : (int)threadIdx.x / T;
+        const int64_t r = min(r0 + row, rows - 1);  // rows past the end are not stored
+        base = KC ? p + r * ld + E * kg : p + E * kg * ld + r;
+        step = KC ? BK : BK * ld;
+        fast = !KC || (ld % 4 == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0);
+    }
+    // Stage i of the first term (whole, vector loads).
+    __device__ __forceinline__ void load_fast(int64_t i, int64_t ld, float* x) const {
+        const float* q = base + i * step;
+        if constexpr (KC) {
+#pragma unroll
+            for (int v = 0; v < E / 4; ++v) {
+                const f32x4 u = reinterpret_cast<const f32x4*>(q)[v];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * v + e] = u[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[e] = q[e * ld];
+        }
+    }
+    // k in [k0, k0 + BK) of any operand, element by element: the last stage
+    // of a term, unaligned rows, the second term.
+    __device__ __forceinline__ void load_any(const float* p, int64_t ld, bool kc, int64_t r0, int64_t rows, int64_t k0,
+                                             int64_t K, float* x) const {
+        const int64_t sr = kc ? ld : 1, sk = kc ? 1 : ld, k = k0 + E * kg;
+        const float* q = p + min(r0 + row, rows - 1) * sr;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const float v = q[min(k + e, K - 1) * sk];
+            x[e] = k + e < K ? v : 0.f;
+        }
+    }
+    __device__ __forceinline__ void store(uint4* lds, const float* x) const {
+        const Split<E> s = split3<E>(x);
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p) {
+            uint4* d = lds + p * T * BK / 8 + chunk_at<BK>(row, E * kg / 8);
+            if constexpr (E == 8)
+                *d = make_uint4(s.p[p][0], s.p[p][1], s.p[p][2], s.p[p][3]);
+            else
+                reinterpret_cast<uint2*>(d)[kg & 1] = make_uint2(s.p[p][0], s.p[p][1]);
+        }
+    }
+};
+
+// This term's part of element (m, n) over k in [k0, k1), in plain fp32.
+__device__ __forceinline__ float exact_dot(const GemmF32Term& f, int64_t m, int64_t n, int64_t k0, int64_t k1,
+                                           float sum) {
+    const int64_t am = f.ta ? 1 : f.lda, ak = f.ta ? f.lda : 1, bn = f.tb ? f.ldb : 1, bk = f.tb ? 1 : f.ldb;
+    for (int64_t k = k0; k < min(k1, f.K); ++k) sum = fmaf(f.alpha * f.A[m * am + k * ak], f.B[n * bn + k * bk], sum);
+    return sum;
+}
+
+// TA / TB: term 0's storage.  KW groups of 2 x 2 waves share a stage's 16-deep
+// k steps; their accumulators are added through LDS at the end.
+template <int T, int BK, int KW, bool TA, bool TB>
+__global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
+    constexpr int MT = T / 64, NT = T / 64;  // 32 x 32 tiles per wave
+    constexpr int kThreads = 256 * KW, KS = BK / 16 / KW;  // k steps of a wave per stage
+    constexpr int TM = T, TN = T, kBuf = kPlanes * T * BK / 8;  // uint4 per operand and buffer
+    __shared__ uint4 lds[4 * kBuf];  // [buffer][A, B]
+    const int lane = threadIdx.x & 63, w = wave_id(), n = lane & 31, hh = lane >> 5;
+    const int wm = w & 1, wn = w >> 1 & 1, wk = w >> 2;
+
+    // Tiles that share the larger operand's rows run next to each other on one
+    // XCD: the smaller tile count fastest, then the other, then the k slices.
+    int i = xcd_block((int)blockIdx.x, (int)gridDim.x);
+    const int per = a.tiles_m * a.tiles_n, slice = i / per;
+    i -= slice * per;
+    const bool m_fast = a.tiles_m <= a.tiles_n;
+    const int tm = m_fast ? i % a.tiles_m : i / a.tiles_n, tn = m_fast ? i / a.tiles_m : i % a.tiles_n;
+    const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
+    const int s0 = slice * a.per_slice, s1 = min(s0 + a.per_slice, a.stages);
+
+    const GemmF32Term &f = a.g.terms[0], &h = a.g.terms[1];
+    Loader<T, BK, kThreads, !TA> ldr_a;
+    Loader<T, BK, kThreads, TB> ldr_b;
+    constexpr int E = decltype(ldr_a)::E;
+    ldr_a.init(f.A, f.lda, m0, a.g.M);
+    ldr_b.init(f.B, f.ldb, n0, a.g.N);
+    // Stages [s0, sf) are whole and go by vector loads.
+    const int sf = ldr_a.fast && ldr_b.fast && f.alpha == 1.f ? max(s0, min(s1, (int)(f.K / BK))) : s0;
+    f32x16 acc[NT][MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int k = 0; k < MT; ++k) {
+            acc[j][k] = zero16();
+            asm volatile("" : "+v"(acc[j][k]));  // not a literal zero (see mfma_v_first)
+        }
+    struct Operands {
+        bf16x8 a[KS][MT][kPlanes], b[KS][NT][kPlanes];
+    };
+    auto read = [&](int buf) {
+        const uint4* la = lds + buf * 2 * kBuf;
+        const uint4* lb = la + kBuf;
+        Operands o;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p) {
+#pragma unroll
+                for (int k = 0; k < MT; ++k)
+                    o.a[ks][k][p] = __builtin_bit_cast(
+                        bf16x8, la[p * T * BK / 8 + chunk_at<BK>(wm * (TM / 2) + 32 * k + n, 2 * (KS * wk + ks) + hh)]);
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    o.b[ks][j][p] = __builtin_bit_cast(
+                        bf16x8, lb[p * T * BK / 8 + chunk_at<BK>(wn * (TN / 2) + 32 * j + n, 2 * (KS * wk + ks) + hh)]);
+            }
+        return o;
+    };
+    // C^T = B^T A^T per 32 x 32 tile (four consecutive n per register group),
+    // the smallest products first.
+    auto multiply = [&](const Operands& o) {
+        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int k = 0; k < MT; ++k)
+                        acc[j][k] = mfma_bf16(o.b[ks][j][pb[q]], o.a[ks][k][pa[q]], acc[j][k]);
+    };
+    float xa[2][E], xb[2][E];
+    auto fetch = [&](int s, float* u, float* v) {  // a fast stage; past the last one, that again
+        const int64_t i = min(s, sf - 1);
+        ldr_a.load_fast(i, f.lda, u);
+        ldr_b.load_fast(i, f.ldb, v);
+    };
+    // Stage s from LDS buffer `buf`, while stage s + 1 goes from registers to
+    // the other buffer; stage s + 3 is then loaded in its place.  No branch
+    // inside: the compiler's waits then count the loads of each stage.
+    auto step = [&](int s, int buf, float* u, float* v) {
+        const Operands o = read(buf);
+        uint4* next = lds + (buf ^ 1) * 2 * kBuf;
+        multiply(o);
+        ldr_a.store(next, u);
+        ldr_b.store(next + kBuf, v);
+#pragma unroll
+        for (int q = 0; q < 6 * MT * NT * KS; ++q) {  // the split between the MFMAs
+            __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(SG_VALU, MT * NT > 1 ? 4 : 8, 0);
+        }
+        fetch(s + 3, u, v);
+        lds_barrier();
+    };
+    if (s0 < sf) {
+        fetch(s0, xa[0], xb[0]);
+        fetch(s0 + 1, xa[1], xb[1]);
+        ldr_a.store(lds, xa[0]);
+        ldr_b.store(lds + kBuf, xb[0]);
+        fetch(s0 + 2, xa[0], xb[0]);
+        lds_barrier();
+        for (int s = s0; s < sf; s += 2) {
+            step(s, 0, xa[1], xb[1]);
+            if (s + 1 < sf) step(s + 1, 1, xa[0], xb[0]);
+        }
+    }
+    // The other stages one at a time: a term's last, partial one, the second
+    // term's, and all of operands that vector loads do not fit.
+    for (int s = sf; s < s1; ++s) {
+        const bool second = s >= a.n0;
+        const int64_t k0 = (int64_t)BK * (second ? s - a.n0 : s), K = second ? h.K : f.K;
+        const float alpha = second ? h.alpha : f.alpha;
+        ldr_a.load_any(second ? h.A : f.A, second ? h.lda : f.lda, second ? h.ta == 0 : !TA, m0, a.g.M, k0, K, xa[0]);
+        ldr_b.load_any(second ? h.B : f.B, second ? h.ldb : f.ldb, second ? h.tb != 0 : TB, n0, a.g.N, k0, K, xb[0]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) xa[0][e] *= alpha;
+        lds_barrier();
+        ldr_a.store(lds, xa[0]);
+        ldr_b.store(lds + kBuf, xb[0]);
+        lds_barrier();
+        multiply(read(0));
+    }
+
+    if constexpr (KW > 1) {
+        static_assert(KW == 2 && MT * NT == 1, "two groups of waves, one 32 x 32 tile each");
+        float* other = reinterpret_cast<float*>(lds) + (w & 3) * 16 * 64 + lane;
+        lds_barrier();
+        if (wk == 1)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) other[64 * r] = acc[0][0][r];
+        lds_barrier();
+        if (wk == 1) return;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][0][r] += other[64 * r];
+    }
+    float* C = a.whole ? a.g.C : a.g.partial + (int64_t)slice * a.g.M * a.g.N;
+    const int64_t ldc = a.whole ? a.g.ldc : a.g.N;
+    const float* bias = a.whole ? a.g.bias : nullptr;
+    const bool vec = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+    const int64_t mw = m0 + wm * (TM / 2) + n, nw = n0 + wn * (TN / 2) + 4 * hh;
+    bool nan = false;
+#pragma unroll
+    for (int k = 0; k < MT; ++k) {
+        const int64_t m = mw + 32 * k;
+        if (m >= a.g.M) continue;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t c0 = nw + 32 * j + 8 * q;
+                f32x4 o{acc[j][k][4 * q], acc[j][k][4 * q + 1], acc[j][k][4 * q + 2], acc[j][k][4 * q + 3]};
+                float* d = C + m * ldc + c0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    nan |= o[e] != o[e];
+                    if (bias && c0 + e < a.g.N) o[e] += bias[c0 + e];
+                }
+                if (vec && c0 + 4 <= a.g.N) {
+                    *reinterpret_cast<f32x4*>(d) = o;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (c0 + e < a.g.N) d[e] = o[e];
+                }
+            }
+    }
+    if (!nan) return;
+    // This lane's elements once more, those that are NaN in plain fp32.
+    for (int i = 0; i < 16 * MT * NT; ++i) {
+        const int64_t m = mw + 32 * (i / (16 * NT)), c = nw + 32 * (i / 16 % NT) + 8 * (i / 4 % 4) + i % 4;
+        if (m >= a.g.M || c >= a.g.N) continue;
+        float* d = C + m * ldc + c;
+        if (*d == *d) continue;
+        const int64_t e0 = min(s0, a.n0), e1 = min(s1, a.n0);
+        float x = exact_dot(a.g.terms[0], m, c, (int64_t)BK * e0, (int64_t)BK * e1, 0.f);
+        x = exact_dot(a.g.terms[1], m, c, (int64_t)BK * (s0 - e0), (int64_t)BK * (s1 - e1), x);
+        *d = x + (bias ? bias[c] : 0.f);
+    }
+}
+
+// C (+)= the slices' partial products in slice order, + bias.
+template <int VEC>
+__global__ __launch_bounds__(256) void gemm_f32_reduce(Args a) {
+    typedef float V __attribute__((ext_vector_type(VEC)));
+    const int64_t MN = a.g.M * a.g.N, i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
+    if (i >= MN) return;
+    const int64_t m = i / a.g.N, n = i - m * a.g.N;  // N is a multiple of VEC
+    V sum = *reinterpret_cast<const V*>(a.g.partial + i);
+#pragma unroll 8
+    for (int s = 1; s < a.slices; ++s) sum += *reinterpret_cast<const V*>(a.g.partial + s * MN + i);
+    float* d = a.g.C + m * a.g.ldc + n;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) d[e] = sum[e] + (a.g.bias ? a.g.bias[n + e] : 0.f) + (a.g.add ? d[e] : 0.f);
+}
+
+struct Plan {
+    bool small;  // 64 x 64 tiles
+    Args a;
+};
+
+// 128 x 128 tiles where they fill the GPU, with k cut into slices or
+// not; else 64 x 64.  k is cut into slices of at least kMinSlice values until
+// about two workgroups per CU run, where the tiles alone leave more than half
+// of the GPU idle (each slice costs an fp32 tile written and read again).
+constexpr int kMinSlice = 256;
+Plan plan(const GemmF32& g) {
+    Plan p{};
+    const int cus = device_cus();
+    auto tiles = [&](int t) { return ((g.M + t - 1) / t) * ((g.N + t - 1) / t); };
+    const int64_t K = g.terms[0].K + g.terms[1].K;
+    auto cut = [&](int64_t t) {
+        return 2 * t >= cus ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / t, K / kMinSlice));
+    };
+    p.small = tiles(128) * cut(tiles(128)) < cus;
+    const int t = p.small ? 64 : 128, bk = p.small ? 32 : 16;
+    p.a.g = g;
+    p.a.tiles_m = (int)((g.M + t - 1) / t);
+    p.a.tiles_n = (int)((g.N + t - 1) / t);
+    p.a.n0 = (int)((g.terms[0].K + bk - 1) / bk);
+    const int stages = p.a.stages = p.a.n0 + (int)((g.terms[1].K + bk - 1) / bk);
+    const int slices = cut(tiles(t));
+    p.a.per_slice = (stages + slices - 1) / slices;
+    p.a.slices = (stages + p.a.per_slice - 1) / p.a.per_slice;
+    p.a.whole = p.a.slices == 1 && !g.add;
+    return p;
+}
+
+template <int T, int BK, int KW>
+void launch_t(const Args& a, hipStream_t st) {
+    const dim3 grid((unsigned)(a.tiles_m * a.tiles_n * a.slices));
+    const bool ta = a.g.terms[0].ta != 0, tb = a.g.terms[0].tb != 0;
+    if (ta && tb)
+        hipLaunchKernelGGL((gemm_f32_kernel<T, BK, KW, true, true>), grid, dim3(256 * KW), 0, st, a);
+    else if (ta)
+        hipLaunchKernelGGL((gemm_f32_kernel<T, BK, KW, true, false>), grid, dim3(256 * KW), 0, st, a);
+    else if (tb)
+        hipLaunchKernelGGL((gemm_f32_kernel<T, BK, KW, false, true>), grid, dim3(256 * KW), 0, st, a);
+    else
+        hipLaunchKernelGGL((gemm_f32_kernel<T, BK, KW, false, false>), grid, dim3(256 * KW), 0, st, a);
+}
+
+}  // namespace
+
+size_t gemm_f32_workspace(const GemmF32& g) {
+    const Plan p = plan(g);
+    return !p.a.whole ? (size_t)p.a.slices * g.M * g.N * 4 : 0;
+}
+
+hipError_t launch_gemm_f32(const GemmF32& g, hipStream_t st) {
+    if (g.M <= 0 || g.N <= 0) return hipSuccess;
+    const Plan p = plan(g);
+    if (p.small)
+        launch_t<64, 32, 2>(p.a, st);
+    else
+        launch_t<128, 16, 1>(p.a, st);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || p.a.whole) return e;
+    const int64_t MN = g.M * g.N;
+    if (g.N % 4 == 0)
+        hipLaunchKernelGGL(gemm_f32_reduce<4>, dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0, st, p.a);
+    else
+        hipLaunchKernelGGL(gemm_f32_reduce<1>, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, st, p.a);
+    return hipGetLastError();
+}
+
+}  // namespace mft

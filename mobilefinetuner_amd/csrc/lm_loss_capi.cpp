@@ -3,8 +3,8 @@
 // Validation mirrors the reference's checks (core/lm_loss.cpp:273-286 for the
 // dense variant, :389-414 for the selected-token / streaming variant).  The
 // streaming variant cuts the vocabulary into chunks of `chunk` rows of the
-// LM-head weight; per chunk, with rocBLAS column-major GEMMs over the
-// row-major tensors:
+// LM-head weight; per chunk, with fp32 GEMMs on the bf16 matrix units
+// (gemm_f32.h) or, for bf16 operands, rocBLAS:
 //   forward   Z = hidden . W_c^T          (fp32 [N, chunk], workspace)
 //             row statistics of Z merged into the running (max, sum)
 //   backward  Z recomputed, G = (exp(Z - lse) - onehot) * coeff  (input dtype)
@@ -16,10 +16,12 @@
 // straight from the recomputed logits (no fp32 chunk).
 #include "mft/lm_loss.h"
 
+#include <algorithm>
 #include <string>
 
 #include "blas_util.h"
 #include "capi_util.h"
+#include "gemm_f32.h"
 #include "lm_loss_kernels.h"
 
 namespace {
@@ -27,6 +29,11 @@ namespace {
 using namespace mft::capi;
 
 constexpr int64_t kDefaultChunk = 16384;
+// fp32: the default chunk grows while a chunk's logits stay within 128 MiB
+// (half of the last-level cache), so that few positions do not run GEMMs too
+// short to fill the GPU: forward and backward at 512 positions, a vocabulary of
+// 50257 and H 768 take 966 us as one chunk and 1060 as four.
+constexpr int64_t kDefaultLogits = int64_t(1) << 25;
 constexpr size_t kBlasWorkspace = size_t(64) << 20;
 
 size_t up(size_t x) { return (x + 255) & ~size_t(255); }
@@ -36,8 +43,43 @@ struct Layout {
 };
 
 int64_t chunk_of(const mft_lm_loss_desc* d) {
-    const int64_t c = d->chunk > 0 ? d->chunk : kDefaultChunk;
+    int64_t c = d->chunk > 0 ? d->chunk : kDefaultChunk;
+    if (d->chunk == 0 && d->dtype == MFT_F32) c = std::max(c, kDefaultLogits / (d->B * d->S));
     return c < d->V ? c : d->V;
+}
+
+// Row stride of a chunk's logits and G: a multiple of 8 elements, so that
+// every row takes vector loads and stores (at a vocabulary of 50257 in one
+// chunk the fp32 G . W took 431 us on unaligned rows, 248 on aligned ones).
+int64_t chunk_ld(int64_t chunk) { return (chunk + 7) / 8 * 8; }
+
+// The three products of a chunk of nc vocabulary rows in fp32:
+// Z[N, nc] = hidden . W_c^T (row stride ldg), grad_hidden (+)= G . W_c, grad_W_c = G^T . hidden.
+struct ChunkGemms {
+    mft::GemmF32 z, dh, dw;
+};
+ChunkGemms chunk_gemms(const mft_lm_loss_desc* d, int64_t nc, int64_t ldg) {
+    const int64_t N = d->B * d->S, H = d->H;
+    ChunkGemms c{};
+    c.z.M = N, c.z.N = nc, c.z.ldc = ldg;
+    c.z.terms[0] = {nullptr, nullptr, H, H, H, 0, 1, 1.f};
+    c.dh.M = N, c.dh.N = H, c.dh.ldc = H, c.dh.add = 1;
+    c.dh.terms[0] = {nullptr, nullptr, ldg, H, nc, 0, 0, 1.f};
+    c.dw.M = nc, c.dw.N = H, c.dw.ldc = H;
+    c.dw.terms[0] = {nullptr, nullptr, ldg, H, N, 1, 0, 1.f};
+    return c;
+}
+// Their workspace, for whole chunks and the last one.
+size_t chunk_gemms_workspace(const mft_lm_loss_desc* d, int64_t chunk) {
+    size_t w = 0;
+    for (const int64_t nc : {chunk, d->V % chunk ? d->V % chunk : chunk}) {
+        const ChunkGemms c = chunk_gemms(d, nc, chunk_ld(chunk));
+        for (const mft::GemmF32* g : {&c.z, &c.dh, &c.dw}) w = std::max(w, mft::gemm_f32_workspace(*g));
+        mft::GemmF32 first = c.dh;  // the first chunk's is not added to anything
+        first.add = 0;
+        w = std::max(w, mft::gemm_f32_workspace(first));
+    }
+    return w;
 }
 
 Layout layout(const mft_lm_loss_desc* d, bool streaming) {
@@ -52,12 +94,11 @@ Layout layout(const mft_lm_loss_desc* d, bool streaming) {
     if (streaming) {
         const size_t c = (size_t)chunk_of(d);
         const size_t esz = d->dtype == MFT_BF16 ? 2 : 4;
-        // the fused kernels need no fp32 logits chunk; their G rows are
-        // padded to a multiple of 8 elements (8-byte stores)
+        // the fused kernels need no fp32 logits chunk
         const bool fused = mft::ce_fused_supported(d->H, d->dtype == MFT_BF16);
-        l.z = o, o += fused ? 0 : up(N * c * 4);
-        l.g = o, o += up(N * (fused ? (c + 7) / 8 * 8 : c) * esz);
-        l.blas = o, o += kBlasWorkspace;
+        l.z = o, o += fused ? 0 : up(N * chunk_ld((int64_t)c) * 4);
+        l.g = o, o += up(N * chunk_ld((int64_t)c) * esz);
+        l.blas = o, o += d->dtype == MFT_F32 ? up(chunk_gemms_workspace(d, (int64_t)c)) : kBlasWorkspace;
         // fused forward: (max, sum) pairs per position and vocabulary part
         l.part = o, o += up(N * 2 * mft::kCeFusedMaxRanges * sizeof(float2));
     }
@@ -104,14 +145,59 @@ mft::CeArgs args(const mft_lm_loss_desc* d, const Layout& l, void* ws, const int
     return a;
 }
 
-// Z[N, nc] (row-major, fp32) = hidden[N, H] . W[v0 : v0 + nc, :]^T
-mft_status logits_chunk(rocblas_handle h, const mft_lm_loss_desc* d, const void* hidden, const void* weight,
-                        int64_t v0, int64_t nc, float* Z) {
-    const bool bf = d->dtype == MFT_BF16;
-    const char* W = static_cast<const char*>(weight) + v0 * d->H * (bf ? 2 : 4);
-    return mft::blas::gemm_rm("mft_lm_ce", h, d->B * d->S, nc, d->H, 1.f, hidden, d->H, false, W, d->H, true, 0.f, Z,
-                              nc, bf);
-}
+// The streaming variant's GEMMs of one call: gemm_f32 for fp32 operands, one
+// rocBLAS handle (locked for the call) for bf16.
+class Gemms {
+public:
+    Gemms(const mft_lm_loss_desc* d, const void* hidden, char* ws, hipStream_t st)
+        : d_(d), hidden_(hidden), ws_(ws), st_(st), bf_(d->dtype == MFT_BF16), N_(d->B * d->S), H_(d->H) {}
+    mft_status begin(const char* who) {
+        who_ = who;
+        if (!bf_) return MFT_OK;
+        lock_ = mft::blas::lock();
+        return mft::blas::bind(who, st_, ws_, kBlasWorkspace, &h_);
+    }
+    // Z[N, nc] (row stride ldz, fp32) = hidden[N, H] . W[v0 : v0 + nc, :]^T
+    mft_status logits(const void* weight, int64_t v0, int64_t nc, float* Z, int64_t ldz) {
+        const char* W = static_cast<const char*>(weight) + v0 * H_ * (bf_ ? 2 : 4);
+        if (bf_)
+            return mft::blas::gemm_rm(who_, h_, N_, nc, H_, 1.f, hidden_, H_, false, W, H_, true, 0.f, Z, ldz, true);
+        return run(chunk_gemms(d_, nc, ldz).z, hidden_, W, Z);
+    }
+    // gh[N, H] (+)= G[N, nc] . W_c[nc, H]
+    mft_status grad_hidden(const void* G, int64_t ldg, const void* Wc, int64_t nc, bool add, float* gh) {
+        if (bf_)
+            return mft::blas::gemm_rm(who_, h_, N_, H_, nc, 1.f, G, ldg, false, Wc, H_, false, add ? 1.f : 0.f, gh, H_,
+                                      true);
+        mft::GemmF32 g = chunk_gemms(d_, nc, ldg).dh;
+        g.add = add;
+        return run(g, G, Wc, gh);
+    }
+    // gw[nc, H] = G^T . hidden
+    mft_status grad_weight(const void* G, int64_t ldg, int64_t nc, float* gw) {
+        if (bf_)
+            return mft::blas::gemm_rm(who_, h_, nc, H_, N_, 1.f, G, ldg, true, hidden_, H_, false, 0.f, gw, H_, true);
+        return run(chunk_gemms(d_, nc, ldg).dw, G, hidden_, gw);
+    }
+
+private:
+    mft_status run(mft::GemmF32 g, const void* A, const void* B, float* C) {
+        g.terms[0].A = static_cast<const float*>(A);
+        g.terms[0].B = static_cast<const float*>(B);
+        g.C = C;
+        g.partial = reinterpret_cast<float*>(ws_);
+        return hip_status(mft::launch_gemm_f32(g, st_), who_);
+    }
+    const mft_lm_loss_desc* d_;
+    const void* hidden_;
+    char* ws_;
+    hipStream_t st_;
+    bool bf_;
+    int64_t N_, H_;
+    const char* who_ = "";
+    std::unique_lock<std::mutex> lock_;
+    rocblas_handle h_ = nullptr;
+};
 
 }  // namespace
 
@@ -182,14 +268,13 @@ mft_status mft_lm_ce_streaming_fwd(const mft_lm_loss_desc* desc, const void* hid
         return hip_status(e, "mft_lm_ce_streaming_fwd launch");
     }
     float* Z = reinterpret_cast<float*>(w + l.z);
-    const int64_t chunk = chunk_of(desc);
-    auto lock = mft::blas::lock();
-    rocblas_handle h;
-    if ((r = mft::blas::bind("mft_lm_ce_streaming_fwd", stream, w + l.blas, kBlasWorkspace, &h)) != MFT_OK) return r;
+    const int64_t chunk = chunk_of(desc), ldz = chunk_ld(chunk);
+    Gemms gemms(desc, hidden, w + l.blas, stream);
+    if ((r = gemms.begin("mft_lm_ce_streaming_fwd")) != MFT_OK) return r;
     for (int64_t v0 = 0; v0 < desc->V; v0 += chunk) {
         const int64_t nc = desc->V - v0 < chunk ? desc->V - v0 : chunk;
-        if ((r = logits_chunk(h, desc, hidden, weight, v0, nc, Z)) != MFT_OK) return r;
-        const hipError_t e = mft::launch_ce_stats(a, Z, false, nc, nc, v0, v0 == 0, stream);
+        if ((r = gemms.logits(weight, v0, nc, Z, ldz)) != MFT_OK) return r;
+        const hipError_t e = mft::launch_ce_stats(a, Z, false, ldz, nc, v0, v0 == 0, stream);
         if (e != hipSuccess) return hip_status(e, "mft_lm_ce_streaming_fwd launch");
     }
     return hip_status(mft::launch_ce_finalize(a, stream), "mft_lm_ce_streaming_fwd launch");
@@ -215,11 +300,10 @@ mft_status mft_lm_ce_streaming_bwd(const mft_lm_loss_desc* desc, const void* hid
     const int64_t chunk = chunk_of(desc), N = desc->B * desc->S, H = desc->H;
     hipError_t e = mft::launch_ce_count(a, stream);
     if (e != hipSuccess) return hip_status(e, "mft_lm_ce_streaming_bwd launch");
-    auto lock = mft::blas::lock();
-    rocblas_handle h;
-    if ((r = mft::blas::bind("mft_lm_ce_streaming_bwd", stream, w + l.blas, kBlasWorkspace, &h)) != MFT_OK) return r;
+    Gemms gemms(desc, hidden, w + l.blas, stream);
+    if ((r = gemms.begin("mft_lm_ce_streaming_bwd")) != MFT_OK) return r;
     const bool fused = mft::ce_fused_supported(H, bf);
-    const int64_t ldg = fused ? (chunk + 7) / 8 * 8 : chunk;
+    const int64_t ldg = chunk_ld(chunk);
     mft::CeFusedArgs plan{};
     for (int64_t v0 = 0; v0 < desc->V; v0 += chunk) {
         const int64_t nc = desc->V - v0 < chunk ? desc->V - v0 : chunk;
@@ -228,18 +312,12 @@ mft_status mft_lm_ce_streaming_bwd(const mft_lm_loss_desc* desc, const void* hid
             if (v0 == 0 || nc != chunk) plan = mft::ce_fused_plan(N, nc, H);
             e = mft::launch_ce_fused_grad(a, plan, hidden, Wc, v0, G, ldg, stream);
         } else {
-            if ((r = logits_chunk(h, desc, hidden, weight, v0, nc, Z)) != MFT_OK) return r;
-            e = mft::launch_ce_grad(a, Z, false, nc, nc, v0, G, bf, ldg, stream);
+            if ((r = gemms.logits(weight, v0, nc, Z, ldg)) != MFT_OK) return r;
+            e = mft::launch_ce_grad(a, Z, false, ldg, nc, v0, G, bf, ldg, stream);
         }
         if (e != hipSuccess) return hip_status(e, "mft_lm_ce_streaming_bwd launch");
-        // grad_hidden[N, H] (+)= G[N, nc] . W_c[nc, H]
-        if (grad_hidden && (r = mft::blas::gemm_rm("mft_lm_ce_streaming_bwd", h, N, H, nc, 1.f, G, ldg, false, Wc, H,
-                                                   false, v0 > 0 ? 1.f : 0.f, grad_hidden, H, bf)) != MFT_OK)
-            return r;
-        // grad_weight[v0 : v0 + nc, :] = G^T . hidden
-        if (grad_weight && (r = mft::blas::gemm_rm("mft_lm_ce_streaming_bwd", h, nc, H, N, 1.f, G, ldg, true, hidden,
-                                                   H, false, 0.f, grad_weight + v0 * H, H, bf)) != MFT_OK)
-            return r;
+        if (grad_hidden && (r = gemms.grad_hidden(G, ldg, Wc, nc, v0 > 0, grad_hidden)) != MFT_OK) return r;
+        if (grad_weight && (r = gemms.grad_weight(G, ldg, nc, grad_weight + v0 * H)) != MFT_OK) return r;
     }
     return MFT_OK;
 }

@@ -302,3 +302,44 @@ def test_dense_unaligned_rows(dev, case):
     assert torch.allclose(loss.double().view(-1), ref.reshape(-1), rtol=1e-5, atol=0)
     assert torch.allclose(lse.double().view(-1), torch.where(on, ref_lse, 0.0), rtol=1e-5, atol=0)
     assert float((grad.double().view(B * S, V) - rg).abs().max()) <= 2e-6 * float(rg.abs().max())
+
+
+@pytest.mark.parametrize("case", [
+    (1, 2, 16, 64, 0),        # one tile, one k step
+    (1, 65, 33, 257, 0),      # rows that vector loads do not fit, tiles of one row
+    (2, 100, 768, 4099, 0),   # k cut into slices
+    (1, 129, 48, 1000, 250),  # chunks of unequal length added to grad_hidden
+    (3, 43, 640, 20001, 0),   # wide tiles, an odd vocabulary in one chunk
+], ids=lambda c: "B{}S{}H{}V{}-c{}".format(*c))
+def test_streaming_fp32_products(dev, case):
+    """The fp32 products at the edges of their tiles and k stages, against
+    double precision.  Six bf16 products stand for one fp32 product to 2^-21
+    at worst and the sums are fp32: 4e-6 of the norm (a plain fp32 product of
+    the largest of these has 2e-6), 1e-5 for the loss and lse."""
+    import torch
+    from mobilefinetuner_amd import lm_loss as L
+    B, S, H, V, chunk = case
+    print(f"[case] fp32 products {case}", flush=True)
+    g = torch.Generator(device=dev)
+    g.manual_seed(V + H)
+    h = 0.5 * torch.randn(B, S, H, device=dev, generator=g)
+    w = 0.2 * torch.randn(V, H, device=dev, generator=g)
+    y = torch.randint(0, V, (B, S), device=dev, generator=g, dtype=torch.int32)
+    loss, lse = L.streaming_lm_cross_entropy(h, w, y, -100, "sum", chunk)
+    gh, gw = L.streaming_lm_cross_entropy_backward(h, w, y, lse, torch.ones(1, device=dev), -100, "sum", chunk)
+    h64, w64 = h.double().view(-1, H), w.double()
+    t = torch.full((B, S), -100, dtype=torch.int64, device=dev)
+    t[:, :-1] = y[:, 1:]
+    t = t.view(-1)
+    on = t >= 0
+    z = h64 @ w64.T
+    ref_lse = torch.logsumexp(z, 1)
+    nll = (ref_lse - z.gather(1, t.clamp(min=0)[:, None])[:, 0])[on].sum()
+    p = (z - ref_lse[:, None]).exp()
+    p[torch.arange(B * S, device=dev), t.clamp(min=0)] -= 1.0
+    p *= on[:, None]
+    errs = [float((a.double().reshape(b.shape) - b).norm() / b.norm()) for a, b in ((gh, p @ w64), (gw, p.T @ h64))]
+    print(f"[errs] {errs}", flush=True)
+    assert abs(float(loss) - float(nll)) <= 1e-5 * abs(float(nll))
+    assert torch.allclose(lse.double().view(-1), torch.where(on, ref_lse, 0.0), rtol=1e-5, atol=1e-6)
+    assert max(errs) <= 4e-6, errs
