@@ -44,11 +44,12 @@ using namespace bwd;
 // Row terms of a query row for the P recompute, in log2 units:
 // P = exp2(x * lc - t0 - t1).  Plain: x is the raw dot product, lc =
 // scale * log2(e), t0 = lse * log2(e), t1 = 0.  Mask mode: x is the
-// mask_score (natural units), lc = log2(e), (t0, t1) = (row max, ln sum) *
+// masked score (natural units), lc = log2(e), (t0, t1) = (row max, ln sum) *
 // log2(e) from the forward's lse pair; x * lc - t0 is exactly 0 at the row
 // max, so a uniform row (all scores equal and huge) still gets P = 1 / n.
 template <bool MASK>
 __device__ __forceinline__ void row_terms(const float* lse, int64_t ri, bool valid, float* t0, float* t1) {
+#pragma clang fp contract(off)
     if constexpr (MASK) {
         *t0 = valid ? lse[2 * ri] * kLog2e : INFINITY;
         *t1 = valid ? lse[2 * ri + 1] * kLog2e : 0.f;
@@ -56,6 +57,15 @@ __device__ __forceinline__ void row_terms(const float* lse, int64_t ri, bool val
         *t0 = valid ? lse[ri] * kLog2e : INFINITY;
         *t1 = 0.f;
     }
+}
+
+// P in mask mode.  Each step rounded on its own: a fused x * log2(e) - t0
+// would leave the product's rounding error, up to 512 at x = -1e10.
+__device__ __forceinline__ float mask_p(float x, float t0, float t1) {
+#pragma clang fp contract(off)
+    const float y = x * kLog2e;
+    const float z = y - t0;
+    return fast_exp2(z - t1);
 }
 
 // ------------------------------------------------------------------ DELTA
@@ -188,6 +198,8 @@ __device__ __forceinline__ void dkdv_bf16_body(const BwdArgs& a, char* smem, int
             }
             // lane column n = key; register r = query qb + row_of_reg(r, hh)
             const bool need_mask = !vis.all(qb, qb + 31, wkey0, wkey0 + 31);
+            if constexpr (MASK)
+                mask_scores16<false>(s, a.scale, a.mask_causal, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const f32x4 l4 = *reinterpret_cast<const f32x4*>(Ls + 8 * g + 4 * hh);
@@ -198,11 +210,7 @@ __device__ __forceinline__ void dkdv_bf16_body(const BwdArgs& a, char* smem, int
                     const int r = 4 * g + i;
                     float p;
                     if constexpr (MASK) {
-                        const int qr = qb + 8 * g + 4 * hh + i;
-                        const float x = qr < S && key < S
-                                            ? mask_score(s[r], a.scale, a.mask_causal, a.m0, a.m1, b, h, qr, key)
-                                            : -INFINITY;
-                        p = fast_exp2((x * kLog2e - l4[i]) - e4[i]);
+                        p = mask_p(s[r], l4[i], e4[i]);
                     } else {
                         p = fast_exp2(s[r] * a.scale_log2 - l4[i]);
                         if (need_mask && !vis.visible(qb + 8 * g + 4 * hh + i, key)) p = 0.f;
@@ -337,6 +345,8 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdArgs& a, char* smem, int 
                 }
             }
             const bool need_mask = !vis.all(qb, qb + 31, wkey0, wkey0 + 31);
+            if constexpr (MASK)
+                mask_scores16<false>(s, a.scale, a.mask_causal, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const f32x4 l4 = *reinterpret_cast<const f32x4*>(Ls + 8 * g + 4 * hh);
@@ -347,11 +357,7 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdArgs& a, char* smem, int 
                     const int r = 4 * g + i;
                     float p;
                     if constexpr (MASK) {
-                        const int qr = qb + 8 * g + 4 * hh + i;
-                        const float x = qr < S && key < S
-                                            ? mask_score(s[r], a.scale, a.mask_causal, a.m0, a.m1, b, h, qr, key)
-                                            : -INFINITY;
-                        p = fast_exp2((x * kLog2e - l4[i]) - e4[i]);
+                        p = mask_p(s[r], l4[i], e4[i]);
                     } else {
                         p = fast_exp2(s[r] * a.scale_log2 - l4[i]);
                         if (need_mask && !vis.visible(qb + 8 * g + 4 * hh + i, key)) p = 0.f;
@@ -489,15 +495,14 @@ __device__ __forceinline__ void dq_body(const BwdArgs& a, char* smem, int qt, in
                 }
             }
             // lane column n = query row; register r = key kbase + 32kk + row_of_reg(r, hh)
+            if constexpr (MASK)
+                mask_scores16<true>(s, a.scale, a.mask_causal, a.m0, a.m1, b, h, row, kbase + 32 * kk + 4 * hh, S);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = kbase + 32 * kk + row_of_reg(r, hh);
                 float p;
                 if constexpr (MASK) {
-                    const float x = row < S && key < S
-                                        ? mask_score(s[r], a.scale, a.mask_causal, a.m0, a.m1, b, h, row, key)
-                                        : -INFINITY;
-                    p = fast_exp2((x * kLog2e - lse2) - lse2b);
+                    p = mask_p(s[r], lse2, lse2b);
                 } else {
                     p = fast_exp2(s[r] * a.scale_log2 - lse2);
                     if (need_mask && !vis.visible(row, key)) p = 0.f;
@@ -598,7 +603,7 @@ hipError_t launch_bwd_t(const AttnShape& s, BwdArgs a, int stages, hipStream_t s
         constexpr int NW = BF ? 4 : f32_dkdv_warps(DP), BN = BF ? 64 : f32_dq_bn(DP);
         const bool kv = stages & BWD_STAGE_DKDV, q = stages & BWD_STAGE_DQ;
         // (causal, mask mode) -> instantiation; mask mode applies the causal
-        // flag per element (mask_score) and visits every key
+        // flag per element (mask_scores16) and visits every key
 #define MFT_BWD_ROLES(C, M)                                                                                     \
     do {                                                                                                        \
         if constexpr (BF) {                                                                                     \
@@ -725,18 +730,19 @@ int dkdv_keys_per_block(const AttnShape& s) {
 }
 
 int dkdv_splits(const AttnShape& s) {
-    // Split the query heads of a group across workgroups until the whole
-    // MAIN grid (dK/dV blocks + dQ blocks) has about one workgroup per CU;
-    // splits must divide the group size.
+    // Split the query heads of a group across workgroups until the dK/dV
+    // launch has about one workgroup per CU (the general kernels run a launch
+    // per role); splits must divide the group size.  Counted together with the
+    // dQ blocks, B 4, Hq 14, Hkv 2, S 512 at D = 64 ran 32 workgroups: 647 us
+    // against @@ with 224 and their REDUCE.
     const int64_t group = s.Hq / s.Hkv;
     const int64_t kb = dkdv_keys_per_block(s);
     const int64_t kv_base = ((s.S + kb - 1) / kb) * s.Hkv * s.B;
-    const int64_t q_blocks = s.bf16 ? ((s.S + 127) / 128) * s.Hq * s.B : 0;
     int64_t best = 1;
     for (int64_t d = 1; d <= group; ++d) {
         if (group % d) continue;
         best = d;
-        if (kv_base * d + q_blocks >= 256) break;
+        if (kv_base * d >= 256) break;
     }
     return (int)best;
 }

@@ -49,7 +49,7 @@ template <typename T, int DP, int BN> struct FwdLds {
 };
 
 // MASK: mask mode (AttnShape::masked, CAUSAL false): every key, scores from
-// mask_score, the running max in natural units, and lse written as the pair
+// mask_scores16, the running max in natural units, and lse written as the pair
 // (row max, ln sum), which keeps the row's sum exact when its scores are
 // huge (a row masked by -1e10 everywhere is a uniform softmax).
 template <typename T, int DP, int NW, int BN, bool CAUSAL, bool MASK = false>
@@ -163,14 +163,13 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(FwdArgs a) {
         float mx = -INFINITY;
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
+            if constexpr (MASK)  // a row past the end takes the last row's scores; it is not stored
+                mask_scores16<true>(s[kk], a.scale, a.mask_causal, a.m0, a.m1, b, h, rowc, kbase + 32 * kk + 4 * hh, S);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 float x = s[kk][r];
                 const int key = kbase + 32 * kk + row_of_reg(r, hh);
-                if constexpr (MASK)
-                    x = key < S ? mask_score(x, a.scale, a.mask_causal, a.m0, a.m1, b, h, rowc, key) : -INFINITY;
-                else if (need_mask && !vis.visible(row, key))
-                    x = -INFINITY;
+                if (!MASK && need_mask && !vis.visible(row, key)) x = -INFINITY;
                 s[kk][r] = x;
                 mx = fmaxf(mx, x);
             }
@@ -341,7 +340,7 @@ hipError_t launch_fwd_t(const AttnShape& s, FwdArgs a, hipStream_t st) {
     constexpr int BM = 32 * NW;
     a.n_qtiles = (int)((s.S + BM - 1) / BM);
     dim3 grid(a.n_qtiles, (unsigned)s.Hq, (unsigned)s.B);
-    if (s.masked)  // causal or not: mask_score applies the flag per element
+    if (s.masked)  // causal or not: mask_scores16 applies the flag per element
         hipLaunchKernelGGL((attn_fwd_kernel<T, DP, NW, BN, false, true>), grid, dim3(NW * 64), 0, st, a);
     else if (s.causal)
         hipLaunchKernelGGL((attn_fwd_kernel<T, DP, NW, BN, true>), grid, dim3(NW * 64), 0, st, a);

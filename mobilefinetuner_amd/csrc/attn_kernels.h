@@ -25,24 +25,72 @@ struct Strides {
 struct MaskView {
     const float* p;
     int64_t sb, sh, si, sj;
-    __host__ __device__ float at(int64_t b, int64_t h, int64_t i, int64_t j) const {
-        return p[b * sb + h * sh + i * si + j * sj];
-    }
 };
 
-// The score of (query row i, key j) of batch b, query head h in mask mode,
-// with the reference's float operations in their order: dot * scale, replaced
-// by -1e10 above the diagonal when causal (the no-grad operator,
-// core/memory_efficient_attention.cpp:160-172), then + mask0 and + mask1 (the
-// composite's mul then add, :29-38; the model graphs' base then padding mask,
-// graph/gemma_model.cpp:494-499).  No fused multiply-add: the reference rounds
-// each step.
-__device__ __forceinline__ float mask_score(float dot, float scale, int causal, const MaskView& m0,
-                                            const MaskView& m1, int b, int h, int i, int j) {
-    float x = (causal && j > i) ? -1e10f : __fmul_rn(dot, scale);
-    if (m0.p) x = __fadd_rn(x, m0.at(b, h, i, j));
-    if (m1.p) x = __fadd_rn(x, m1.at(b, h, i, j));
-    return x;
+// One mask's values at the 16 accumulator elements of a lane, all loads in
+// flight together.  KEYS: the lane has query row i, its elements keys j +
+// row_of_reg(r, 0); else key j and rows i + row_of_reg(r, 0) (the caller adds
+// its half-wave's offset to j or i).  whole: every element is inside [0, S);
+// else indices are clamped.  Keys next to each other in memory are read four
+// at a time where their rows start on 16 bytes.
+template <bool KEYS>
+__device__ __forceinline__ void mask_load16(const MaskView& m, int b, int h, int i, int j, int S, bool whole,
+                                            float (&v)[16]) {
+    const float* base = m.p + b * m.sb + h * m.sh;
+    const int64_t step = KEYS ? m.sj : m.si;
+    if (whole) {
+        const float* p = base + i * m.si + j * m.sj;
+        if (KEYS && m.sj == 1 && ((m.sb | m.sh | m.si) & 3) == 0 && (reinterpret_cast<uintptr_t>(m.p) & 15) == 0) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float4 x = *reinterpret_cast<const float4*>(p + 8 * g);  // j is a multiple of 4
+                v[4 * g] = x.x, v[4 * g + 1] = x.y, v[4 * g + 2] = x.z, v[4 * g + 3] = x.w;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = p[(8 * (r >> 2) + (r & 3)) * step];
+        }
+    } else {
+        const int n0 = KEYS ? j : i;
+        const float* p = base + (KEYS ? i * m.si : j * m.sj);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = p[min(n0 + 8 * (r >> 2) + (r & 3), S - 1) * step];
+    }
+}
+
+// The scores of a lane's 16 elements in mask mode (elements as in
+// mask_load16), in place of the dot products, with the reference's float
+// operations in their order: dot * scale, replaced by -1e10 above the diagonal
+// when causal (the no-grad operator, core/memory_efficient_attention.cpp:
+// 160-172), then + mask0 and + mask1 (the composite's mul then add, :29-38;
+// the model graphs' base then padding mask, graph/gemma_model.cpp:494-499).
+// Nothing is contracted: the reference rounds each step.  Elements outside
+// [0, S) become -inf.
+template <bool KEYS, class Acc>
+__device__ __forceinline__ void mask_scores16(Acc& s, float scale, int causal, const MaskView& m0, const MaskView& m1,
+                                              int b, int h, int i, int j, int S) {
+#pragma clang fp contract(off)
+    const bool whole = KEYS ? j + 28 <= S : i + 28 <= S;
+    float v0[16], v1[16];
+    const int ic = KEYS ? min(i, S - 1) : i, jc = KEYS ? j : min(j, S - 1);
+    if (m0.p) mask_load16<KEYS>(m0, b, h, ic, jc, S, whole, v0);
+    if (m1.p) mask_load16<KEYS>(m1, b, h, ic, jc, S, whole, v1);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int n = 8 * (r >> 2) + (r & 3), ir = KEYS ? i : i + n, jr = KEYS ? j + n : j;
+        s[r] = (causal && jr > ir) ? -1e10f : s[r] * scale;
+    }
+    if (m0.p)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] += v0[r];
+    if (m1.p)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] += v1[r];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int n = 8 * (r >> 2) + (r & 3), ir = KEYS ? i : i + n, jr = KEYS ? j + n : j;
+        if (ir >= S || jr >= S) s[r] = -INFINITY;
+    }
 }
 
 struct AttnShape {
