@@ -178,6 +178,11 @@ __device__ __forceinline__ void dkdv_bf16_body(const BwdArgs& a, char* smem, int
                     Dl[tid] = r < S ? dl[r] : 0.f;
                 }
             }
+            // With the block's own loads, where registers allow (65 -> 59 us at the
+            // shape of dkdv_splits; in the forward and the dQ role, whose lanes are
+            // rows, the same slowed the tile's loads: 37 -> 54 and 43 -> 60 us).
+            MaskVals mv;
+            if constexpr (MASK && DP <= 128) mask_fetch16<false>(mv, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
             __syncthreads();
             if (wkey0 >= S) continue;  // no valid keys in this wave
             // no row of the block sees a key of this wave
@@ -198,8 +203,10 @@ __device__ __forceinline__ void dkdv_bf16_body(const BwdArgs& a, char* smem, int
             }
             // lane column n = key; register r = query qb + row_of_reg(r, hh)
             const bool need_mask = !vis.all(qb, qb + 31, wkey0, wkey0 + 31);
-            if constexpr (MASK)
-                mask_scores16<false>(s, a.scale, a.mask_causal, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
+            if constexpr (MASK) {
+                if constexpr (DP > 128) mask_fetch16<false>(mv, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
+                mask_scores16<false>(s, mv, a.scale, a.mask_causal, a.m0, a.m1, qb + 4 * hh, key, S);
+            }
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const f32x4 l4 = *reinterpret_cast<const f32x4*>(Ls + 8 * g + 4 * hh);
@@ -325,6 +332,8 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdArgs& a, char* smem, int 
                     Dl[tid] = r < S ? dl[r] : 0.f;
                 }
             }
+            MaskVals mv;  // with the block's own loads (see the bf16 body)
+            if constexpr (MASK && DP <= 128) mask_fetch16<false>(mv, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
             __syncthreads();
             if (wkey0 >= S) continue;
             if (!vis.any(qb, min(qb + 31, S - 1), wkey0, min(wkey0 + 31, S - 1))) continue;
@@ -345,8 +354,10 @@ __device__ __forceinline__ void dkdv_f32_body(const BwdArgs& a, char* smem, int 
                 }
             }
             const bool need_mask = !vis.all(qb, qb + 31, wkey0, wkey0 + 31);
-            if constexpr (MASK)
-                mask_scores16<false>(s, a.scale, a.mask_causal, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
+            if constexpr (MASK) {
+                if constexpr (DP > 128) mask_fetch16<false>(mv, a.m0, a.m1, b, h, qb + 4 * hh, key, S);
+                mask_scores16<false>(s, mv, a.scale, a.mask_causal, a.m0, a.m1, qb + 4 * hh, key, S);
+            }
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const f32x4 l4 = *reinterpret_cast<const f32x4*>(Ls + 8 * g + 4 * hh);
@@ -495,8 +506,12 @@ __device__ __forceinline__ void dq_body(const BwdArgs& a, char* smem, int qt, in
                 }
             }
             // lane column n = query row; register r = key kbase + 32kk + row_of_reg(r, hh)
-            if constexpr (MASK)
-                mask_scores16<true>(s, a.scale, a.mask_causal, a.m0, a.m1, b, h, row, kbase + 32 * kk + 4 * hh, S);
+            if constexpr (MASK) {
+                const int key0 = kbase + 32 * kk + 4 * hh;
+                MaskVals mv;
+                mask_fetch16<true>(mv, a.m0, a.m1, b, h, row, key0, S);
+                mask_scores16<true>(s, mv, a.scale, a.mask_causal, a.m0, a.m1, row, key0, S);
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int key = kbase + 32 * kk + row_of_reg(r, hh);
@@ -734,7 +749,7 @@ int dkdv_splits(const AttnShape& s) {
     // launch has about one workgroup per CU (the general kernels run a launch
     // per role); splits must divide the group size.  Counted together with the
     // dQ blocks, B 4, Hq 14, Hkv 2, S 512 at D = 64 ran 32 workgroups: 647 us
-    // against @@ with 224 and their REDUCE.
+    // against 59 with 224, and 5 of REDUCE.
     const int64_t group = s.Hq / s.Hkv;
     const int64_t kb = dkdv_keys_per_block(s);
     const int64_t kv_base = ((s.S + kb - 1) / kb) * s.Hkv * s.B;

@@ -163,8 +163,12 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd_kernel(FwdArgs a) {
         float mx = -INFINITY;
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
-            if constexpr (MASK)  // a row past the end takes the last row's scores; it is not stored
-                mask_scores16<true>(s[kk], a.scale, a.mask_causal, a.m0, a.m1, b, h, rowc, kbase + 32 * kk + 4 * hh, S);
+            if constexpr (MASK) {  // a row past the end takes the last row's scores; it is not stored
+                const int key0 = kbase + 32 * kk + 4 * hh;
+                MaskVals mv;
+                mask_fetch16<true>(mv, a.m0, a.m1, b, h, rowc, key0, S);
+                mask_scores16<true>(s[kk], mv, a.scale, a.mask_causal, a.m0, a.m1, rowc, key0, S);
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 float x = s[kk][r];

@@ -58,6 +58,19 @@ __device__ __forceinline__ void mask_load16(const MaskView& m, int b, int h, int
     }
 }
 
+// Both masks' values at a lane's 16 elements, loaded before they are needed.
+struct MaskVals {
+    float v0[16], v1[16];
+};
+template <bool KEYS>
+__device__ __forceinline__ void mask_fetch16(MaskVals& v, const MaskView& m0, const MaskView& m1, int b, int h, int i,
+                                             int j, int S) {
+    const bool whole = KEYS ? j + 28 <= S : i + 28 <= S;
+    const int ic = KEYS ? min(i, S - 1) : i, jc = KEYS ? j : min(j, S - 1);
+    if (m0.p) mask_load16<KEYS>(m0, b, h, ic, jc, S, whole, v.v0);
+    if (m1.p) mask_load16<KEYS>(m1, b, h, ic, jc, S, whole, v.v1);
+}
+
 // The scores of a lane's 16 elements in mask mode (elements as in
 // mask_load16), in place of the dot products, with the reference's float
 // operations in their order: dot * scale, replaced by -1e10 above the diagonal
@@ -67,14 +80,9 @@ __device__ __forceinline__ void mask_load16(const MaskView& m, int b, int h, int
 // Nothing is contracted: the reference rounds each step.  Elements outside
 // [0, S) become -inf.
 template <bool KEYS, class Acc>
-__device__ __forceinline__ void mask_scores16(Acc& s, float scale, int causal, const MaskView& m0, const MaskView& m1,
-                                              int b, int h, int i, int j, int S) {
+__device__ __forceinline__ void mask_scores16(Acc& s, const MaskVals& v, float scale, int causal, const MaskView& m0,
+                                              const MaskView& m1, int i, int j, int S) {
 #pragma clang fp contract(off)
-    const bool whole = KEYS ? j + 28 <= S : i + 28 <= S;
-    float v0[16], v1[16];
-    const int ic = KEYS ? min(i, S - 1) : i, jc = KEYS ? j : min(j, S - 1);
-    if (m0.p) mask_load16<KEYS>(m0, b, h, ic, jc, S, whole, v0);
-    if (m1.p) mask_load16<KEYS>(m1, b, h, ic, jc, S, whole, v1);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int n = 8 * (r >> 2) + (r & 3), ir = KEYS ? i : i + n, jr = KEYS ? j + n : j;
@@ -82,10 +90,10 @@ __device__ __forceinline__ void mask_scores16(Acc& s, float scale, int causal, c
     }
     if (m0.p)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] += v0[r];
+        for (int r = 0; r < 16; ++r) s[r] += v.v0[r];
     if (m1.p)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] += v1[r];
+        for (int r = 0; r < 16; ++r) s[r] += v.v1[r];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int n = 8 * (r >> 2) + (r & 3), ir = KEYS ? i : i + n, jr = KEYS ? j + n : j;
