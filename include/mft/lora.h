@@ -21,7 +21,8 @@
  * infers these from the shapes, nn/lora_linear.cpp:52-88).  Slice i adds its
  * [N, cols] delta into columns col0 .. col0 + cols - 1 of y.
  *
- * Arithmetic.  W fp32: every GEMM is an fp32 rocBLAS GEMM.  W bf16: the
+ * Arithmetic.  W fp32: fp32 GEMMs on the bf16 matrix units, each operand as the
+ * exact sum of three bf16 numbers (csrc/gemm_f32.hip).  W bf16: the
  * products with W run on the bf16 MFMA path (x, resp. dy, rounded to bf16 to
  * nearest even; fp32 accumulation); the LoRA branch stays fp32.
  *
@@ -32,8 +33,8 @@
  * that behaviour; 1 gives every slice its gradient.
  *
  * Conventions are those of mft/attention.h (status codes, mft_last_error,
- * caller-owned device memory, stream ordering).  The GEMMs run through
- * rocBLAS on a per-device handle created on first use, with the GEMM
+ * caller-owned device memory, stream ordering).  The bf16 GEMMs that are not
+ * fused run through rocBLAS on a per-device handle created on first use, with the GEMM
  * workspace taken from the caller's workspace.
  */
 #ifndef MFT_LORA_H

@@ -2,6 +2,8 @@
 //
 // The layer is GEMMs plus element-wise staging.  Row-major throughout, R =
 // sum of the slices' ranks, s_i = scale_i:
+//   (fp32 W: y and dx are one product each on the bf16 matrix units, the
+//    update of one slice and the bias with it; gemm_f32.h)
 //   forward   y  = x . W (+ bias)                 rocBLAS; bf16 W: x staged
 //                                                  to bf16 by the first rowdot
 //                                                  (bf16 W [out, in] with one
@@ -31,6 +33,7 @@
 #include "attn_kernels.h"
 #include "blas_util.h"
 #include "capi_util.h"
+#include "gemm_f32.h"
 #include "lm_loss_kernels.h"
 #include "lora_kernels.h"
 
@@ -95,13 +98,15 @@ size_t pack_bytes(const mft_lora_desc* d) {
     return up(m);
 }
 
+size_t products_workspace(const mft_lora_desc* d, bool backward);
+
 FwdLayout fwd_layout(const mft_lora_desc* d) {
     FwdLayout l{};
     size_t o = 0;
     l.xb = o, o += d->w_dtype == MFT_BF16 ? up((size_t)d->N * d->in_dim * 2) : 0;
     l.u = o, o += up((size_t)d->N * total_rank(d) * 4);
     l.pt = o, o += pack_bytes(d);
-    l.blas = o, o += kBlasWorkspace;
+    l.blas = o, o += d->w_dtype == MFT_BF16 ? kBlasWorkspace : products_workspace(d, false);
     l.total = o;
     return l;
 }
@@ -123,7 +128,7 @@ BwdLayout bwd_layout(const mft_lora_desc* d) {
     }
     l.part = o, o += up((size_t)part * 4);
     l.pt = o, o += pack_bytes(d);
-    l.blas = o, o += kBlasWorkspace;
+    l.blas = o, o += d->w_dtype == MFT_BF16 ? kBlasWorkspace : products_workspace(d, true);
     l.total = o;
     return l;
 }
@@ -153,6 +158,66 @@ mft_status coldot(const float* M, int64_t ldm, int64_t rows, int64_t K, const fl
                   const char* who) {
     mft::LoraColDot a{M, ldm, rows, K, V, ldv, (int)r, alpha, partial, out, ok, oj};
     return hip_status(mft::launch_lora_coldot(a, stream), who);
+}
+
+// y [N, out] (fp32 W): x . W + bias, and the update scale u_i . B_i of one slice
+// that spans every column as the same product's second term (slice -1: none).
+// u's column block of the slice is given.
+mft::GemmF32 y_product(const mft_lora_desc* d, int slice, const float* u, int64_t R) {
+    mft::GemmF32 g{};
+    g.M = d->N, g.N = d->out_dim, g.ldc = d->out_dim;
+    g.terms[0] = {nullptr, nullptr, d->in_dim, d->w_transposed ? d->in_dim : d->out_dim, d->in_dim, 0,
+                  d->w_transposed != 0, 1.f};
+    if (slice >= 0) {
+        const mft_lora_slice& s = d->slices[slice];
+        g.terms[1] = {u, s.B, R, s.b_transposed ? s.rank : s.cols, s.rank, 0, s.b_transposed != 0, s.scale};
+    }
+    return g;
+}
+// dx [N, in] (fp32 W): dy . W^T, and g_i . A_i^T of one slice.
+mft::GemmF32 dx_product(const mft_lora_desc* d, int slice, const float* g_i, int64_t R) {
+    mft::GemmF32 g{};
+    g.M = d->N, g.N = d->in_dim, g.ldc = d->in_dim;
+    g.terms[0] = {nullptr, nullptr, d->out_dim, d->w_transposed ? d->in_dim : d->out_dim, d->out_dim, 0,
+                  d->w_transposed == 0, 1.f};
+    if (slice >= 0) {
+        const mft_lora_slice& s = d->slices[slice];
+        g.terms[1] = {g_i, s.A, R, s.a_transposed ? d->in_dim : s.rank, s.rank, 0, s.a_transposed == 0, 1.f};
+    }
+    return g;
+}
+// A further slice's update alone: the second term of `g`, added to C.
+mft::GemmF32 update_only(mft::GemmF32 g) {
+    g.terms[0] = g.terms[1];
+    g.terms[1] = {};
+    g.add = 1;
+    return g;
+}
+
+// The first slice whose update joins the main product: of the forward one
+// that spans every column, of the backward one that has gradients.
+int joined_slice(const mft_lora_desc* d, bool backward) {
+    for (int i = 0; i < d->n_slices; ++i) {
+        const mft_lora_slice& s = d->slices[i];
+        if (backward ? has_grad(d, s) : s.col0 == 0 && s.cols == d->out_dim) return i;
+    }
+    return -1;
+}
+
+// Workspace of the fp32 products of one direction (never 0: the calls take no
+// NULL workspace).
+size_t products_workspace(const mft_lora_desc* d, bool backward) {
+    const int64_t R = total_rank(d);
+    const int j = joined_slice(d, backward);
+    auto product = backward ? dx_product : y_product;
+    size_t w = std::max<size_t>(256, mft::gemm_f32_workspace(product(d, j, nullptr, R)));
+    for (int i = 0; i < d->n_slices; ++i) {
+        if (i == j) continue;
+        mft::GemmF32 g = update_only(product(d, i, nullptr, R));
+        if (!backward) g.N = d->slices[i].cols;
+        w = std::max(w, mft::gemm_f32_workspace(g));
+    }
+    return up(w);
 }
 
 // op(W) as the right operand of x . W ([in, out]) or of dy . W^T ([out, in]).
@@ -211,7 +276,7 @@ mft_status mft_lora_fwd(const mft_lora_desc* desc, const float* x, const void* W
     mft::CeFusedArgs plan{};
     const bool fused = lora_fused_fwd_ok(desc, &plan);
     hipError_t e = hipSuccess;
-    if (bias && !fused) e = mft::launch_lora_fill_bias(y, bias, N, out, stream);
+    if (bias && bf && !fused) e = mft::launch_lora_fill_bias(y, bias, N, out, stream);
     // bf16 W: the GEMM reads x rounded to bf16, written by the first slice's
     // rowdot (one read of x) or, without slices, by lora_round_bf16.
     uint16_t* xb = bf ? reinterpret_cast<uint16_t*>(ws + l.xb) : nullptr;
@@ -248,12 +313,36 @@ mft_status mft_lora_fwd(const mft_lora_desc* desc, const float* x, const void* W
         return hip_status(mft::launch_lora_fused_fwd(plan, stream), "mft_lora_fwd launch");
     }
 
+    if (!bf) {
+        const int j = joined_slice(desc, false);
+        ro = 0;
+        for (int i = 0; i < j; ++i) ro += desc->slices[i].rank;
+        mft::GemmF32 g = y_product(desc, j, u + ro, R);
+        g.terms[0].A = x;
+        g.terms[0].B = static_cast<const float*>(W);
+        g.C = y;
+        g.bias = bias;
+        g.partial = reinterpret_cast<float*>(ws + l.blas);
+        e = mft::launch_gemm_f32(g, stream);
+        ro = 0;
+        for (int i = 0; e == hipSuccess && i < desc->n_slices; ro += desc->slices[i].rank, ++i) {
+            if (i == j) continue;
+            // y[:, col0 .. col0 + cols] += scale * u_i . B_i
+            mft::GemmF32 s = update_only(y_product(desc, i, u + ro, R));
+            s.N = desc->slices[i].cols;
+            s.C = y + desc->slices[i].col0;
+            s.partial = g.partial;
+            e = mft::launch_gemm_f32(s, stream);
+        }
+        return hip_status(e, "mft_lora_fwd launch");
+    }
+
     auto lock = mft::blas::lock();
     rocblas_handle h;
     if ((r = mft::blas::bind(who, stream, ws + l.blas, kBlasWorkspace, &h)) != MFT_OK) return r;
     const WOperand wo = w_for_forward(desc);
-    if ((r = mft::blas::gemm_rm(who, h, N, out, in, 1.f, bf ? static_cast<const void*>(xb) : x, in, false, W, wo.ld,
-                                wo.t, bias ? 1.f : 0.f, y, out, bf)) != MFT_OK)
+    if ((r = mft::blas::gemm_rm(who, h, N, out, in, 1.f, xb, in, false, W, wo.ld, wo.t, bias ? 1.f : 0.f, y, out,
+                                true)) != MFT_OK)
         return r;
     ro = 0;
     for (int i = 0; i < desc->n_slices; ++i) {
@@ -295,11 +384,6 @@ mft_status mft_lora_bwd(const mft_lora_desc* desc, const float* x, const void* W
         const hipError_t e = mft::launch_lora_round_bf16(dy, dyb, N * out, stream);
         if (e != hipSuccess) return hip_status(e, "mft_lora_bwd launch");
     }
-    const void* dyo = dyb ? static_cast<const void*>(dyb) : dy;
-
-    auto lock = mft::blas::lock();
-    rocblas_handle h;
-    if ((r = mft::blas::bind(who, stream, ws + l.blas, kBlasWorkspace, &h)) != MFT_OK) return r;
     int64_t ro = 0;
     for (int i = 0; i < desc->n_slices; ++i) {
         const mft_lora_slice& s = desc->slices[i];
@@ -324,8 +408,31 @@ mft_status mft_lora_bwd(const mft_lora_desc* desc, const float* x, const void* W
         ro += rk;
     }
     if (!dx) return MFT_OK;
+    if (!bf) {
+        const int j = joined_slice(desc, true);
+        ro = 0;
+        for (int i = 0; i < j; ++i) ro += desc->slices[i].rank;
+        mft::GemmF32 p = dx_product(desc, j, g + ro, R);
+        p.terms[0].A = dy;
+        p.terms[0].B = static_cast<const float*>(W);
+        p.C = dx;
+        p.partial = reinterpret_cast<float*>(ws + l.blas);
+        hipError_t e = mft::launch_gemm_f32(p, stream);
+        ro = 0;
+        for (int i = 0; e == hipSuccess && i < desc->n_slices; ro += desc->slices[i].rank, ++i) {
+            if (i == j || !has_grad(desc, desc->slices[i])) continue;
+            mft::GemmF32 s = update_only(dx_product(desc, i, g + ro, R));
+            s.C = dx;
+            s.partial = p.partial;
+            e = mft::launch_gemm_f32(s, stream);
+        }
+        return hip_status(e, "mft_lora_bwd launch");
+    }
+    auto lock = mft::blas::lock();
+    rocblas_handle h;
+    if ((r = mft::blas::bind(who, stream, ws + l.blas, kBlasWorkspace, &h)) != MFT_OK) return r;
     const WOperand wo = w_for_backward(desc);
-    if ((r = mft::blas::gemm_rm(who, h, N, in, out, 1.f, dyo, out, false, W, wo.ld, wo.t, 0.f, dx, in, bf)) != MFT_OK)
+    if ((r = mft::blas::gemm_rm(who, h, N, in, out, 1.f, dyb, out, false, W, wo.ld, wo.t, 0.f, dx, in, true)) != MFT_OK)
         return r;
     ro = 0;
     for (int i = 0; i < desc->n_slices; ++i) {
