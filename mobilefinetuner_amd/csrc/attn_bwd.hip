@@ -714,13 +714,16 @@ BwdPlan plan_bwd_fast(const AttnShape& s) {
     return p;
 }
 
-BwdLayout bwd_layout(const AttnShape& s, const BwdPlan& p) {
+namespace {
+
+// The layout with the general kernels' dK/dV cut into `splits` head groups
+// (not read on the fast path).
+BwdLayout layout_of(const AttnShape& s, const BwdPlan& p, int64_t splits) {
     auto up = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
     const size_t rows = static_cast<size_t>(s.B * s.Hq);
     const size_t stat_floats = rows * static_cast<size_t>((s.S + 31) / 32) * 64;
     const size_t delta_floats = rows * static_cast<size_t>(s.S);
     const size_t kv_elems = static_cast<size_t>(s.B * s.Hkv * s.S * s.D);
-    const size_t q_elems = static_cast<size_t>(s.B * s.Hq * s.S * s.D);
     BwdLayout l;
     l.stats = up(sizeof(float) * std::max(stat_floats, delta_floats));
     if (p.fast) {
@@ -730,7 +733,6 @@ BwdLayout bwd_layout(const AttnShape& s, const BwdPlan& p) {
         l.kv_part = p.kv_parts_max > 1 ? up(sizeof(float) * 2 * tile * 2 * p.kv.units * s.B * s.Hkv) : 0;
         l.q_part = p.q_parts_max > 1 ? up(sizeof(float) * tile * 2 * p.q.units * s.B * s.Hq) : 0;
     } else {
-        const int splits = dkdv_splits(s);
         l.kv_part = splits > 1 ? up(sizeof(float) * 2 * splits * kv_elems) : 0;
         l.q_part = 0;
     }
@@ -738,6 +740,10 @@ BwdLayout bwd_layout(const AttnShape& s, const BwdPlan& p) {
     l.total = l.stats + l.kv_part + l.q_part + l.masked;
     return l;
 }
+
+}  // namespace
+
+BwdLayout bwd_layout(const AttnShape& s, const BwdPlan& p) { return layout_of(s, p, p.fast ? 1 : dkdv_splits(s)); }
 
 int dkdv_keys_per_block(const AttnShape& s) {
     if (s.bf16) return 128;
@@ -749,13 +755,19 @@ int dkdv_splits(const AttnShape& s) {
     // launch has about one workgroup per CU (the general kernels run a launch
     // per role); splits must divide the group size.  Counted together with the
     // dQ blocks, B 4, Hq 14, Hkv 2, S 512 at D = 64 ran 32 workgroups: 647 us
-    // against 59 with 224, and 5 of REDUCE.
+    // against 59 with 224, and 5 of REDUCE.  Where dK/dV and dQ together fill
+    // the chip, splits whose partials would take the workspace past the scratch
+    // of the backward without a workspace are left out, so that it still serves
+    // the shape.
     const int64_t group = s.Hq / s.Hkv;
     const int64_t kb = dkdv_keys_per_block(s);
     const int64_t kv_base = ((s.S + kb - 1) / kb) * s.Hkv * s.B;
-    int64_t best = 1;
+    const int64_t q_blocks = s.bf16 ? ((s.S + 127) / 128) * s.Hq * s.B : 0;
+    const BwdPlan general{};
+    int64_t best = 0;
     for (int64_t d = 1; d <= group; ++d) {
         if (group % d) continue;
+        if (best && kv_base * best + q_blocks >= 256 && layout_of(s, general, d).total > kNoAllocScratchBytes) break;
         best = d;
         if (kv_base * d >= 256) break;
     }

@@ -145,7 +145,7 @@ mft_status check_desc(const mft_attn_desc* d, mft::AttnShape* s) {
 // Scratch of mft_attn_bwd_noalloc: the backward workspace (row terms, fp32
 // partial tiles) of callers that cannot allocate.  One copy per GPU, held
 // until the process ends; the host only ever uses its per-device address.
-constexpr size_t kNoAllocScratchBytes = size_t(128) << 20;
+using mft::kNoAllocScratchBytes;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 constexpr int kMaxDevices = 64;

@@ -124,6 +124,8 @@ int fwd_rows_per_block(const AttnShape& s);
 int dkdv_keys_per_block(const AttnShape& s);
 // Number of head groups the dK/dV pass is split into (1 = no partials).
 int dkdv_splits(const AttnShape& s);
+// Scratch of the backward without a workspace (mft_attn_bwd_noalloc).
+constexpr size_t kNoAllocScratchBytes = size_t(128) << 20;
 // The direct-to-LDS kernels with work units: bf16 with D % 8 == 0,
 // 32 < D <= 256 and one K/V sequence stride, and fp32 with D % 4 == 0,
 // 32 < D <= 256 (f32::fast_path).

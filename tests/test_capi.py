@@ -51,6 +51,24 @@ def test_every_header_symbol_is_exported(capi):
         assert hasattr(L, f)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,splits", [
+    (4, 14, 2, 512, 36, 7),     # 32 dK/dV blocks: all seven heads apart
+    (255, 3, 1, 128, 252, 1),   # 255 blocks: three head groups would take 197 MB of partials
+    (63, 64, 1, 512, 252, 1),   # 252 blocks: two groups would take 130 MB, and the row terms 16
+    (63, 4, 1, 512, 252, 2),    # the row terms take 1
+    (300, 4, 1, 128, 36, 1),    # enough blocks unsplit
+    (1, 3, 1, 16384, 252, 3),   # 128 dK/dV and 384 dQ blocks: 99 MB
+])
+def test_general_backward_stays_within_the_fixed_scratch(capi, B, Hq, Hkv, S, D, splits):
+    """bf16 with D % 8 != 0 takes the general kernels; the heads of a group are
+    split over workgroups only where the partials fit mft_attn_bwd_noalloc."""
+    b = capi.workspace_size(capi.desc(B, Hq, Hkv, S, D, 0.125, True, capi.MFT_BF16))[1]
+    partials = 8 * splits * B * Hkv * S * D if splits > 1 else 0
+    terms = 4 * B * Hq * ((S + 31) // 32) * 64
+    assert abs(b - partials - terms) <= 1024
+    assert b <= capi.NOALLOC_SCRATCH_BYTES
+
+
 def test_header_compiles_as_c(tmp_path):
     """The header is plain C (extern "C", C99 types, no torch types)."""
     src = tmp_path / "t.c"
