@@ -187,3 +187,49 @@ def test_reference_errors(dev):
     layer.attach_lora(torch.zeros(8, 2, device=dev), torch.zeros(2, 4, device=dev), 1.0, 4, 4)
     with pytest.raises(RuntimeError, match="exceeds base weight width"):
         layer.forward(torch.zeros(3, 8, device=dev))
+
+
+@pytest.mark.parametrize("N,I,O,wt,specs", [
+    # (rank, scale, col0, cols, a_t, b_t); one element, whole tiles, one past and one short of them
+    (1, 1, 1, False, [(1, 2.0, 0, 1, False, False)]),
+    (128, 128, 256, False, [(8, 2.0, 0, 256, False, False)]),
+    (129, 33, 127, True, [(17, 0.5, 0, 127, True, True)]),
+    (127, 257, 65, False, [(3, 1.0, 0, 65, True, False)]),
+    (300, 70, 516, True, [(4, 2.0, 4, 129, False, True), (5, 1.0, 100, 200, False, False)]),
+    (64, 1040, 40, False, []),
+])
+@pytest.mark.parametrize("inf", [False, True])
+def test_fp32_products_hold_the_fp32_bound(dev, N, I, O, wt, specs, inf):
+    """y and dx with an fp32 W against 64 bits.  A sum of K fp32 products is
+    within (K + 16) 2^-24 of its terms' magnitudes (the six bf16 products of
+    split operands leave out under 2^-21 of them); the update adds its own two
+    sums.  An infinite x gives the infinities and NaN that 64 bits give."""
+    print(f"[case] lora fp32 products {(N, I, O, wt, specs, inf)}", flush=True)
+    rng = np.random.default_rng(N + I + O)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    x, W, bias, dy = f(N, I), f(O, I) if wt else f(I, O), f(O), f(N, O)
+    if inf:
+        x[N // 2, I // 2] = np.inf
+    slices = [dict(A=f(r, I) if at else f(I, r), B=f(c, r) if bt else f(r, c), scale=s, col0=c0,
+                   a_transposed=at, b_transposed=bt) for r, s, c0, c, at, bt in specs]
+    got = _run(dev, x, W, bias, slices, False, dy, True)
+    d = lambda a, t: np.asarray(a.T if t else a, np.float64)
+    x6, W6, dy6 = d(x, False), d(W, wt), d(dy, False)
+    with np.errstate(invalid="ignore"):
+        y, y_mag = x6 @ W6 + bias, np.abs(x6) @ np.abs(W6) + np.abs(bias)
+        dx, dx_mag = dy6 @ W6.T, np.abs(dy6) @ np.abs(W6.T)
+        terms = I + O + 32
+        for s in slices:
+            A6, B6, c = d(s["A"], s["a_transposed"]), d(s["B"], s["b_transposed"]), s["col0"]
+            part = slice(c, c + B6.shape[1])
+            terms += 2 * A6.shape[1]
+            y[:, part] += s["scale"] * ((x6 @ A6) @ B6)
+            y_mag[:, part] += s["scale"] * ((np.abs(x6) @ np.abs(A6)) @ np.abs(B6))
+            dx += s["scale"] * ((dy6[:, part] @ B6.T) @ A6.T)
+            dx_mag += s["scale"] * ((np.abs(dy6[:, part]) @ np.abs(B6.T)) @ np.abs(A6.T))
+    ok = np.isfinite(y)
+    assert ok.all() or inf
+    assert np.array_equal(np.isnan(y), np.isnan(got["y"]))
+    assert np.array_equal(y[np.isinf(y)], got["y"][np.isinf(y)].astype(np.float64))
+    assert (np.abs(got["y"] - y)[ok] <= terms * 2.0 ** -24 * y_mag[ok]).all()
+    assert (np.abs(got["dx"] - dx) <= terms * 2.0 ** -24 * dx_mag).all()
