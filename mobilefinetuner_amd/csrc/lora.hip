@@ -81,9 +81,12 @@ __global__ __launch_bounds__(256) void lora_merge_kernel(LoraMergeArgs a) {
 // block of j at a time), so each P(k, j) it loads serves kRowsPerWg rows.  The
 // 256 partials of each (row, j) are summed through LDS in a fixed order
 // (deterministic).  M is read once per 8-wide block of j: HBM-bound for r <= 8.
+// PV: P is k-contiguous and aligned, so its loads are 16 bytes wide like M's
+// (four times as many 4-byte ones kept the load path busier than M did: [4096
+// x 6912], r 8, with the bf16 copy 52 -> 37 us, 4.6 TB/s).
 constexpr int kRowsPerWg = 8, kJB = 8;
 
-template <int VEC>
+template <int VEC, bool PV>
 __global__ __launch_bounds__(256) void lora_rowdot_kernel(LoraRowDot a) {
     constexpr int NV = kRowsPerWg * kJB;  // partial sums per thread
     __shared__ float red[NV][257];
@@ -99,14 +102,20 @@ __global__ __launch_bounds__(256) void lora_rowdot_kernel(LoraRowDot a) {
         for (int64_t k = (int64_t)VEC * t; k < a.K; k += 256 * VEC) {
             float p[VEC][kJB];
 #pragma unroll
-            for (int v = 0; v < VEC; ++v)
+            for (int j = 0; j < kJB; ++j) {
+                // clamped index, so the load needs no branch; the select zeroes j >= r
+                const int jj = jb + j < a.r ? jb + j : a.r - 1;
+                float pv[VEC];
+                if constexpr (PV) {
+                    const float4 q = *reinterpret_cast<const float4*>(a.P + k + (int64_t)jj * a.pj);
+                    pv[0] = q.x, pv[1 % VEC] = q.y, pv[2 % VEC] = q.z, pv[3 % VEC] = q.w;
+                } else {
 #pragma unroll
-                for (int j = 0; j < kJB; ++j) {
-                    // clamped index, so the load needs no branch; the select zeroes j >= r
-                    const int jj = jb + j < a.r ? jb + j : a.r - 1;
-                    const float pv = a.P[(k + v) * a.pk + (int64_t)jj * a.pj];
-                    p[v][j] = jb + j < a.r ? pv : 0.f;
+                    for (int v = 0; v < VEC; ++v) pv[v] = a.P[(k + v) * a.pk + (int64_t)jj * a.pj];
                 }
+#pragma unroll
+                for (int v = 0; v < VEC; ++v) p[v][j] = jb + j < a.r ? pv[v] : 0.f;
+            }
             float mv[kRowsPerWg][VEC];
 #pragma unroll
             for (int i = 0; i < kRowsPerWg; ++i) {
@@ -163,77 +172,117 @@ __global__ __launch_bounds__(256) void lora_rowdot_kernel(LoraRowDot a) {
     }
 }
 
-// lora_coldot: per chunk c of rows and column k, partial[c][k][j] = sum over
+// lora_coldot: per chunk c of rows and column k, partial[c][j][k] = sum over
 // the chunk's rows of M[n, k] V[n, j]; one wave per (64 VEC columns, chunk),
 // the row of V is the same for the whole wave.  The chunk height is chosen so
 // that about 2048 waves run (lora_coldot_chunk, lora_kernels.h).  Then
-// lora_coldot_reduce sums the chunks in a fixed order.
+// lora_coldot_reduce sums the chunks in a fixed order.  The partials are
+// contiguous in k, a lane's next to its neighbour's (with k outside j each of
+// a wave's 32 stores touched 64 lines), and V comes through scalar loads, a
+// row at a time (M, V and the partials do not overlap; unless the compiler is
+// told, it loads every value of V as a vector).  4096 rows, r 8: K 1152 19.5 ->
+// 10.1 us, K 6912 34.5 -> 20.5, 5.5 TB/s of M.
+
+// acc += M[n, k ..]^T V[n, j0 ..] over rows r0 .. r1 - 1, j < nj (NJ: nj where
+// it is known, so that a row of V is one scalar load; 0 otherwise).
+template <int VEC, int NJ>
+__device__ __forceinline__ void coldot_rows(const float* __restrict__ m, int64_t ldm, const float* __restrict__ V,
+                                            int64_t ldv, int64_t r0, int64_t r1, int nj, float (&acc)[VEC][kJB]) {
+    constexpr int J = NJ ? NJ : kJB;
+#pragma unroll 8
+    for (int64_t n = r0; n < r1; ++n) {
+        const float* row = V + n * ldv;
+        float vv[J];
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const float x = row[NJ || j < nj ? j : nj - 1];
+            vv[j] = NJ || j < nj ? x : 0.f;
+        }
+        float mv[VEC];
+        if (VEC == 4) {
+            const float4 q = *reinterpret_cast<const float4*>(m + n * ldm);
+            mv[0] = q.x, mv[1 % VEC] = q.y, mv[2 % VEC] = q.z, mv[3 % VEC] = q.w;
+        } else {
+            mv[0] = m[n * ldm];
+        }
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+#pragma unroll
+            for (int j = 0; j < J; ++j) acc[v][j] += mv[v] * vv[j];
+    }
+}
 
 template <int VEC>
-__global__ __launch_bounds__(64) void lora_coldot_kernel(LoraColDot a, int64_t chunk) {
+__global__ __launch_bounds__(64) void lora_coldot_kernel(LoraColDot a, const float* __restrict__ M,
+                                                         const float* __restrict__ V, float* __restrict__ partial,
+                                                         int64_t chunk) {
     const int64_t k = ((int64_t)blockIdx.x * 64 + threadIdx.x) * VEC;
     const int64_t c = blockIdx.y;
     const int64_t r0 = c * chunk, r1 = r0 + chunk < a.rows ? r0 + chunk : a.rows;
     const bool live = k < a.K;
+    const float* m = M + (live ? k : 0);  // lanes past K sum a column that they do not store
     for (int jb = 0; jb < a.r; jb += kJB) {
         float acc[VEC][kJB];
 #pragma unroll
         for (int v = 0; v < VEC; ++v)
 #pragma unroll
             for (int j = 0; j < kJB; ++j) acc[v][j] = 0.f;
-#pragma unroll 8
-        for (int64_t n = r0; n < r1; ++n) {
-            float vv[kJB];
+        if (a.r - jb >= kJB)
+            coldot_rows<VEC, kJB>(m, a.ldm, V + jb, a.ldv, r0, r1, kJB, acc);
+        else if (a.r - jb == 4)
+            coldot_rows<VEC, 4>(m, a.ldm, V + jb, a.ldv, r0, r1, 4, acc);
+        else
+            coldot_rows<VEC, 0>(m, a.ldm, V + jb, a.ldv, r0, r1, a.r - jb, acc);
+        if (live) {
+            float* part = partial + (c * a.r + jb) * a.K + k;
 #pragma unroll
             for (int j = 0; j < kJB; ++j) {
-                const int jj = jb + j < a.r ? jb + j : a.r - 1;
-                const float x = a.V[n * a.ldv + jj];
-                vv[j] = jb + j < a.r ? x : 0.f;
+                if (jb + j >= a.r) break;
+                if (VEC == 4)
+                    *reinterpret_cast<float4*>(part + j * a.K) =
+                        make_float4(acc[0][j], acc[1 % VEC][j], acc[2 % VEC][j], acc[3 % VEC][j]);
+                else
+                    part[j * a.K] = acc[0][j];
             }
-            float mv[VEC];
-            if (live) {
-                const float* m = a.M + n * a.ldm + k;
-                if (VEC == 4) {
-                    const float4 q = *reinterpret_cast<const float4*>(m);
-                    mv[0] = q.x, mv[1 % VEC] = q.y, mv[2 % VEC] = q.z, mv[3 % VEC] = q.w;
-                } else {
-                    mv[0] = m[0];
-                }
-            } else {
-#pragma unroll
-                for (int v = 0; v < VEC; ++v) mv[v] = 0.f;
-            }
-#pragma unroll
-            for (int v = 0; v < VEC; ++v)
-#pragma unroll
-                for (int j = 0; j < kJB; ++j) acc[v][j] += mv[v] * vv[j];
-        }
-        if (live) {
-            float* part = a.partial + (c * a.K + k) * a.r + jb;
-#pragma unroll
-            for (int v = 0; v < VEC; ++v)
-#pragma unroll
-                for (int j = 0; j < kJB; ++j)
-                    if (jb + j < a.r) part[v * a.r + j] = acc[v][j];
         }
     }
 }
 
-// Sixteen lanes per output value: lane l sums chunks l, l + 16, ... in order,
-// then the sixteen sums combine in a fixed butterfly (deterministic).
-__global__ __launch_bounds__(256) void lora_coldot_reduce(LoraColDot a, int64_t chunks) {
-    const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) / 16;
-    const int l = threadIdx.x % 16;
-    const int64_t total = a.K * a.r;
+// A workgroup owns 64 consecutive output values; its wave l sums chunks l,
+// l + 8, ... in order, then the eight sums combine in a fixed tree
+// (deterministic).  Eight chunks' loads are in flight together: one after the
+// other they cost a memory round trip each (256 chunks of 1152 x 8 8.0 ->
+// 5.3 us, 64 of 6912 x 8 9.1 -> 5.0).
+constexpr int kColRed = 8;
+__global__ __launch_bounds__(64 * kColRed) void lora_coldot_reduce(LoraColDot a, int64_t chunks) {
+    constexpr int B = 8;
+    __shared__ float sums[kColRed][64];
+    const int le = threadIdx.x % 64, l = threadIdx.x / 64;
+    const int64_t total = a.K * a.r, e = (int64_t)blockIdx.x * 64 + le;
+    const float* src = a.partial + (e < total ? e : total - 1);
     float s = 0.f;
-    if (e < total)
-        for (int64_t c = l; c < chunks; c += 16) s += a.partial[c * total + e];
+    for (int64_t c = l; c < chunks; c += kColRed * B) {
+        float x[B];
 #pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) s += __shfl_xor(s, o, 16);
-    if (e < total && l == 0) {
-        const int64_t k = e / a.r, j = e % a.r;
-        a.out[k * a.ok + j * a.oj] = a.alpha * s;
+        for (int q = 0; q < B; ++q) {
+            const int64_t cq = c + kColRed * q;
+            x[q] = src[(cq < chunks ? cq : chunks - 1) * total];
+        }
+#pragma unroll
+        for (int q = 0; q < B; ++q) s += c + kColRed * q < chunks ? x[q] : 0.f;
     }
+    sums[l][le] = s;
+    __syncthreads();
+    if (l != 0 || e >= total) return;
+    float v[kColRed];
+#pragma unroll
+    for (int i = 0; i < kColRed; ++i) v[i] = sums[i][le];
+#pragma unroll
+    for (int o = kColRed / 2; o >= 1; o >>= 1)
+#pragma unroll
+        for (int i = 0; i < o; ++i) v[i] += v[i + o];
+    const int64_t j = e / a.K, k = e % a.K;
+    a.out[k * a.ok + j * a.oj] = a.alpha * v[0];
 }
 
 __global__ __launch_bounds__(256) void lora_pack_kmajor_kernel(const float* __restrict__ P, int64_t pk, int64_t pj,
@@ -276,10 +325,13 @@ hipError_t launch_lora_rowdot(const LoraRowDot& a, hipStream_t st) {
     const dim3 grid((unsigned)((a.rows + kRowsPerWg - 1) / kRowsPerWg));
     const bool vec = a.K % 4 == 0 && a.ldm % 4 == 0 && (uintptr_t)a.M % 16 == 0 &&
                      (!a.mb || (a.ldb % 4 == 0 && (uintptr_t)a.mb % 8 == 0));
-    if (vec)
-        hipLaunchKernelGGL(lora_rowdot_kernel<4>, grid, dim3(256), 0, st, a);
+    const bool pvec = a.pk == 1 && a.pj % 4 == 0 && (uintptr_t)a.P % 16 == 0;
+    if (vec && pvec)
+        hipLaunchKernelGGL((lora_rowdot_kernel<4, true>), grid, dim3(256), 0, st, a);
+    else if (vec)
+        hipLaunchKernelGGL((lora_rowdot_kernel<4, false>), grid, dim3(256), 0, st, a);
     else
-        hipLaunchKernelGGL(lora_rowdot_kernel<1>, grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((lora_rowdot_kernel<1, false>), grid, dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
@@ -300,15 +352,14 @@ hipError_t launch_lora_coldot(const LoraColDot& a, hipStream_t st) {
     if (a.K <= 0 || a.r <= 0) return hipSuccess;
     const int64_t chunk = lora_coldot_chunk(a.rows, a.K);
     const int64_t chunks = (a.rows + chunk - 1) / chunk;
-    const bool vec = a.K % 4 == 0 && a.ldm % 4 == 0 && (uintptr_t)a.M % 16 == 0;
+    const bool vec = a.K % 4 == 0 && a.ldm % 4 == 0 && (uintptr_t)a.M % 16 == 0 && (uintptr_t)a.partial % 16 == 0;
     const int VEC = vec ? 4 : 1;
     const dim3 grid((unsigned)((a.K + 64 * VEC - 1) / (64 * VEC)), (unsigned)chunks);
     if (vec)
-        hipLaunchKernelGGL(lora_coldot_kernel<4>, grid, dim3(64), 0, st, a, chunk);
+        hipLaunchKernelGGL(lora_coldot_kernel<4>, grid, dim3(64), 0, st, a, a.M, a.V, a.partial, chunk);
     else
-        hipLaunchKernelGGL(lora_coldot_kernel<1>, grid, dim3(64), 0, st, a, chunk);
-    hipLaunchKernelGGL(lora_coldot_reduce, dim3((unsigned)((a.K * a.r * 16 + 255) / 256)), dim3(256), 0, st, a,
-                       chunks);
+        hipLaunchKernelGGL(lora_coldot_kernel<1>, grid, dim3(64), 0, st, a, a.M, a.V, a.partial, chunk);
+    hipLaunchKernelGGL(lora_coldot_reduce, dim3((unsigned)((a.K * a.r + 63) / 64)), dim3(64 * kColRed), 0, st, a, chunks);
     return hipGetLastError();
 }
 

@@ -197,10 +197,12 @@ def test_reference_errors(dev):
     (127, 257, 65, False, [(3, 1.0, 0, 65, True, False)]),
     (300, 70, 516, True, [(4, 2.0, 4, 129, False, True), (5, 1.0, 100, 200, False, False)]),
     (64, 1040, 40, False, []),
+    # 69 chunks of rows in the adapters' gradients, ranks with a remainder of 4 and of 5 after eights
+    (1100, 20, 24, True, [(12, 2.0, 0, 24, True, True), (13, 1.0, 0, 24, False, False)]),
 ])
 @pytest.mark.parametrize("inf", [False, True])
 def test_fp32_products_hold_the_fp32_bound(dev, N, I, O, wt, specs, inf):
-    """y and dx with an fp32 W against 64 bits.  A sum of K fp32 products is
+    """y, dx and the adapters' gradients with an fp32 W against 64 bits.  A sum of K fp32 products is
     within (K + 16) 2^-24 of its terms' magnitudes (the six bf16 products of
     split operands leave out under 2^-21 of them); the update adds its own two
     sums.  An infinite x gives the infinities and NaN that 64 bits give."""
@@ -231,5 +233,12 @@ def test_fp32_products_hold_the_fp32_bound(dev, N, I, O, wt, specs, inf):
     assert ok.all() or inf
     assert np.array_equal(np.isnan(y), np.isnan(got["y"]))
     assert np.array_equal(y[np.isinf(y)], got["y"][np.isinf(y)].astype(np.float64))
-    assert (np.abs(got["y"] - y)[ok] <= terms * 2.0 ** -24 * y_mag[ok]).all()
+    assert (np.abs(got["y"][ok] - y[ok]) <= terms * 2.0 ** -24 * y_mag[ok]).all()
     assert (np.abs(got["dx"] - dx) <= terms * 2.0 ** -24 * dx_mag).all()
+    if not inf:
+        for s, gA, gB in zip(slices, got["grad_A"], got["grad_B"]):
+            A6, B6, c = d(s["A"], s["a_transposed"]), d(s["B"], s["b_transposed"]), s["col0"]
+            part, sc = dy6[:, c:c + B6.shape[1]], s["scale"]
+            for g, t, ref, mag in ((gA, s["a_transposed"], x6.T @ (part @ B6.T), np.abs(x6.T) @ (np.abs(part) @ np.abs(B6.T))),
+                                   (gB, s["b_transposed"], (x6 @ A6).T @ part, (np.abs(x6) @ np.abs(A6)).T @ np.abs(part))):
+                assert (np.abs(d(g, t) - sc * ref) <= (N + terms) * 2.0 ** -24 * sc * mag).all()
