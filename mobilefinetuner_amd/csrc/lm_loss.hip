@@ -13,7 +13,8 @@
 //   ce_finalize   lse = max + log(sum) and nll = lse - z[label] per row, as
 //                 core/lm_loss.cpp:305-312 (double logsumexp)
 //   ce_reduce     scored-row count and the sum of nll in a fixed order
-//                 (double), with ce_finalize's work where rows are few; MEAN divides by the count (NaN if zero), as :345-352
+//                 (double), with the work of ce_finalize where rows are few;
+//                 MEAN divides by the count (NaN if zero), as :345-352
 //   ce_grad       (exp(z - lse) - onehot(label)) * coeff, coeff = grad_loss *
 //                 (1 / count for MEAN), as LMCrossEntropyBackward
 //                 (:85-158): zero rows for unscored positions.

@@ -1,5 +1,5 @@
-// Launchers of the LoRA linear's element-wise kernels (lora.hip; called by
-// lora_capi.cpp).  The GEMMs themselves are rocBLAS calls in lora_capi.cpp.
+// Launchers of the LoRA linear's element-wise and rank-r kernels (lora.hip; called by
+// lora_capi.cpp).  The products with W are gemm_f32 (fp32 W) or rocBLAS calls there.
 #pragma once
 
 #include <hip/hip_runtime.h>
