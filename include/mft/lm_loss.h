@@ -23,9 +23,10 @@
  * GEMM with the online log-sum-exp in its epilogue; no logits are written),
  * and the backward's per-chunk G comes from the same kernel (logits
  * recomputed, G written in bf16).  With fp32 operands the three GEMMs of a
- * chunk run on the bf16 matrix units, each operand as the exact sum of three
- * bf16 numbers (csrc/gemm_f32.hip), with no more rounding than fp32 matrix
- * instructions.  The bf16 backward's two GEMMs per chunk, and the logits GEMMs
+ * chunk run on the bf16 matrix units, each operand as the sum of three bf16
+ * numbers to nearest (csrc/gemm_f32.hip): six of the nine partial products,
+ * the others being under 2^-23.9 of a product and of either sign, so that a sum
+ * is no further from the exact one than fp32 matrix instructions leave it.  The bf16 backward's two GEMMs per chunk, and the logits GEMMs
  * of the other bf16 shapes, run on rocBLAS with a per-device handle created on
  * first use; the GEMM workspace comes from the caller's workspace.
  *

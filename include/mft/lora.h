@@ -21,10 +21,12 @@
  * infers these from the shapes, nn/lora_linear.cpp:52-88).  Slice i adds its
  * [N, cols] delta into columns col0 .. col0 + cols - 1 of y.
  *
- * Arithmetic.  W fp32: fp32 GEMMs on the bf16 matrix units, each operand as the
- * exact sum of three bf16 numbers (csrc/gemm_f32.hip).  W bf16: the
- * products with W run on the bf16 MFMA path (x, resp. dy, rounded to bf16 to
- * nearest even; fp32 accumulation); the LoRA branch stays fp32.
+ * Arithmetic.  W fp32: fp32 GEMMs, the whole stages of 16 or 32 values of k on
+ * the bf16 matrix units with each operand as the sum of three bf16 numbers, the
+ * rest in fp32 matrix instructions; no further from the exact sums than those
+ * are throughout (csrc/gemm_f32.hip).  W bf16: the products
+ * with W run on the bf16 MFMA path (x, resp. dy, rounded to bf16 to nearest
+ * even; fp32 accumulation); the LoRA branch stays fp32.
  *
  * Gradients.  The reference tracks a slice's delta through autograd only when
  * it covers all columns (col0 == 0 and cols == out, nn/lora_linear.cpp:417-

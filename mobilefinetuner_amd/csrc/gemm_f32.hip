@@ -1,18 +1,25 @@
 // fp32 matrix products from bf16 MFMAs.
 //
-// An fp32 number is the exact sum of three bf16 numbers: its top 8 significant
-// bits, the next 8 and the rest (split3, by truncation; both remainders are
-// exact in fp32).  With a = a1 + a2 + a3 and b likewise,
-//   a b = a1 b1 + a1 b2 + a2 b1 + a2 b2 + a1 b3 + a3 b1   (+ terms below 2^-22 a b)
+// An fp32 number is the sum of three bf16 numbers, each the one nearest to what
+// the earlier ones leave (split3; the remainders are exact in fp32, and the
+// last is a bf16 number).  With a = a1 + a2 + a3 and b likewise,
+//   a b = a1 b1 + a1 b2 + a2 b1 + a2 b2 + a1 b3 + a3 b1   (+ a2 b3 + a3 b2 + a3 b3)
 // and each product of two bf16 numbers is exact in the fp32 accumulator's
-// multiplier.  Six v_mfma_f32_32x32x16_bf16 then do the work of eight
+// multiplier.  |a2| <= 2^-8 |a| and |a3| <= 2^-17 |a|: what six products leave
+// out is under 2^-23.9 of a b and as often above as below it (cut to 8 bits
+// each instead of rounded, the parts have the sign of a, and up to 2^-21 is
+// lost towards zero).  Six v_mfma_f32_32x32x16_bf16 do the work of eight
 // v_mfma_f32_32x32x2_f32 in 6 x 32 instead of 8 x 64 cycles, and round the
-// accumulator 6 times per 16 values of k instead of 8.
+// accumulator 6 times per 16 values of k instead of 16.  Those save more than
+// the six products leave out from K = 3 on; what is left of a sum after whole
+// stages of 16 or 32, and with it every shorter sum, goes by fp32 MFMAs.  Norm
+// of the error against 64 bits in 2^-24 of the result, normal operands, beside
+// fp32 MFMAs throughout: K 16 1.0 (1.2), 100 1.7 (3.0), 768 2.9 (8.3); of one
+// sign, 2048 rows: K 768 4.9 (7.1), 4096 9.9 (15.9).
 // What it gives (us, TFLOP/s of the fp32 product; rocBLAS's fp32 kernels beside
 // it): 512 x 16384 x 768 70 us, 183 (96 us); 512 x 768 x 16384 80 us, 161 (124
 // us, 880 without its split-k kernels); 2048 x 16384 x 1024 339 us, 203 (482
-// us), 1.2 PFLOP/s of bf16 products; 509 x 768 x 2304 23 us (21 us).  Error
-// against double precision 0.2 to 0.85 of the fp32 kernels'.  Bound by the
+// us), 1.2 PFLOP/s of bf16 products; 509 x 768 x 2304 23 us (21 us).  Bound by the
 // barrier per stage and the LDS traffic (72 KB per 128 x 128 x 16 stage)
 // beside the MFMAs.
 // Infinities: a remainder of inf, or 0 * inf among the six products, is NaN
@@ -52,25 +59,24 @@ struct Args {
 template <int E> struct Split {
     uint32_t p[kPlanes][E / 2];
 };
-__device__ __forceinline__ uint32_t hi_pair(uint32_t lo, uint32_t hi) {
-    return __builtin_amdgcn_perm(hi, lo, 0x07060302u);  // (hi16 of lo, hi16 of hi)
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {  // to nearest even
+    typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{(bf16)lo, (bf16)hi});
 }
 template <int E> __device__ __forceinline__ Split<E> split3(const float* x) {
     Split<E> s;
 #pragma unroll
     for (int i = 0; i < E / 2; ++i) {
-        uint32_t a[2], b[2], c[2];
+        float lo = x[2 * i], hi = x[2 * i + 1];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const float v = x[2 * i + e];
-            a[e] = __float_as_uint(v);
-            const float r = v - __uint_as_float(a[e] & 0xffff0000u);
-            b[e] = __float_as_uint(r);
-            c[e] = __float_as_uint(r - __uint_as_float(b[e] & 0xffff0000u));
+        for (int p = 0; p < kPlanes; ++p) {
+            // what is left for the last plane is a bf16 number
+            const uint32_t u = p < kPlanes - 1 ? bf16_pair(lo, hi)
+                                               : __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+            s.p[p][i] = u;
+            lo -= __uint_as_float(u << 16);
+            hi -= __uint_as_float(u & 0xffff0000u);
         }
-        s.p[0][i] = hi_pair(a[0], a[1]);
-        s.p[1][i] = hi_pair(b[0], b[1]);
-        s.p[2][i] = hi_pair(c[0], c[1]);
     }
     return s;
 }
@@ -138,6 +144,12 @@ template <int T, int BK, int NT, bool KC> struct Loader {
             else
                 reinterpret_cast<uint2*>(d)[kg & 1] = make_uint2(s.p[p][0], s.p[p][1]);
         }
+    }
+    __device__ __forceinline__ void store_f32(float* lds, int ld, const float* x) const {
+#pragma unroll
+        for (int v = 0; v < E / 4; ++v)
+            *reinterpret_cast<f32x4*>(lds + row * ld + E * kg + 4 * v) =
+                f32x4{x[4 * v], x[4 * v + 1], x[4 * v + 2], x[4 * v + 3]};
     }
 };
 
@@ -240,7 +252,7 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
 #pragma unroll
         for (int q = 0; q < 6 * MT * NT * KS; ++q) {  // the split between the MFMAs
             __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(SG_VALU, MT * NT > 1 ? 4 : 8, 0);
+            __builtin_amdgcn_sched_group_barrier(SG_VALU, MT * NT > 1 ? 5 : 8, 0);
         }
         fetch(s + 3, u, v);
         lds_barrier();
@@ -257,8 +269,15 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
             if (s + 1 < sf) step(s + 1, 1, xa[0], xb[0]);
         }
     }
-    // The other stages one at a time: a term's last, partial one, the second
-    // term's, and all of operands that vector loads do not fit.
+    // The other stages one at a time, in fp32 MFMAs: a term's last, partial
+    // one, the second term's, and all of operands that vector loads do not fit.
+    // Sums of few terms are all here (see the top).  Half hh of a wave takes
+    // values 4 hh .. 4 hh + 3 of each eight k, and the KW groups of waves take
+    // the eights in turn.
+    constexpr int kRow = BK + 4;  // floats from one row to the next
+    float* fa = reinterpret_cast<float*>(lds);
+    float* fb = fa + TM * kRow;
+    static_assert((TM + TN) * kRow * 4 <= sizeof(lds), "a stage in fp32 fits the buffers");
     for (int s = sf; s < s1; ++s) {
         const bool second = s >= a.n0;
         const int64_t k0 = (int64_t)BK * (second ? s - a.n0 : s), K = second ? h.K : f.K;
@@ -268,10 +287,25 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
 #pragma unroll
         for (int e = 0; e < E; ++e) xa[0][e] *= alpha;
         lds_barrier();
-        ldr_a.store(lds, xa[0]);
-        ldr_b.store(lds + kBuf, xb[0]);
+        ldr_a.store_f32(fa, kRow, xa[0]);
+        ldr_b.store_f32(fb, kRow, xb[0]);
         lds_barrier();
-        multiply(read(0));
+        const int eights = (int)min<int64_t>(BK, K - k0 + 7) / 8;
+        for (int i = wk; i < eights; i += KW) {
+            f32x4 va[MT], vb[NT];
+#pragma unroll
+            for (int k = 0; k < MT; ++k)
+                va[k] = *reinterpret_cast<const f32x4*>(fa + (wm * (TM / 2) + 32 * k + n) * kRow + 8 * i + 4 * hh);
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                vb[j] = *reinterpret_cast<const f32x4*>(fb + (wn * (TN / 2) + 32 * j + n) * kRow + 8 * i + 4 * hh);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int k = 0; k < MT; ++k) acc[j][k] = mfma_f32(vb[j][e], va[k][e], acc[j][k]);
+        }
     }
 
     if constexpr (KW > 1) {
