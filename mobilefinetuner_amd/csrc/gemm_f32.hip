@@ -23,8 +23,10 @@
 // barrier per stage and the LDS traffic (72 KB per 128 x 128 x 16 stage)
 // beside the MFMAs.
 // Infinities: a remainder of inf, or 0 * inf among the six products, is NaN
-// where fp32 arithmetic may give inf; an element that comes out NaN is
-// computed again by a plain fp32 dot product (exact_dot).
+// where fp32 arithmetic may give inf.  A tile with a NaN that no NaN operand of
+// its row or column explains is computed again, whole, by the fp32 MFMAs; a NaN
+// operand costs its tiles one more pass over their operands (the LM head and
+// loss at 512 x 768 x 20001 with one NaN 0.75 ms, without 0.46).
 //
 // A workgroup (4 waves) owns a T x T tile of C and a range of BK-deep stages
 // of k (of every term in turn, so that a rank-r update is one or two more
@@ -47,6 +49,9 @@ namespace mft {
 namespace {
 
 constexpr int kPlanes = 3;
+
+// Four floats at any address of a float (the loads take that).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 struct Args {
     GemmF32 g;
@@ -99,9 +104,12 @@ template <int T, int BK, int NT, bool KC> struct Loader {
     const float* base;  // this thread's first element of the fast path
     int64_t step;       // elements from one stage to the next
     bool fast;          // whole stages of the first term go by vector loads
-    __device__ __forceinline__ void init(const float* p, int64_t ld, int64_t r0, int64_t rows) {
-        row = KC ? (int)threadIdx.x / KG : (int)threadIdx.x % T;
-        kg = KC ? (int)threadIdx.x % KG : (int)threadIdx.x / T;
+    __device__ __forceinline__ void place(int tid) {
+        row = KC ? tid / KG : tid % T;
+        kg = KC ? tid % KG : tid / T;
+    }
+    __device__ __forceinline__ void init(int tid, const float* p, int64_t ld, int64_t r0, int64_t rows) {
+        place(tid);
         const int64_t r = min(r0 + row, rows - 1);  // rows past the end are not stored
         base = KC ? p + r * ld + E * kg : p + E * kg * ld + r;
         step = KC ? BK : BK * ld;
@@ -153,22 +161,15 @@ template <int T, int BK, int NT, bool KC> struct Loader {
     }
 };
 
-// This term's part of element (m, n) over k in [k0, k1), in plain fp32.
-__device__ __forceinline__ float exact_dot(const GemmF32Term& f, int64_t m, int64_t n, int64_t k0, int64_t k1,
-                                           float sum) {
-    const int64_t am = f.ta ? 1 : f.lda, ak = f.ta ? f.lda : 1, bn = f.tb ? f.ldb : 1, bk = f.tb ? 1 : f.ldb;
-    for (int64_t k = k0; k < min(k1, f.K); ++k) sum = fmaf(f.alpha * f.A[m * am + k * ak], f.B[n * bn + k * bk], sum);
-    return sum;
-}
-
 // TA / TB: term 0's storage.  KW groups of 2 x 2 waves share a stage's 16-deep
 // k steps; their accumulators are added through LDS at the end.
 template <int T, int BK, int KW, bool TA, bool TB>
-__global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
+__global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
     constexpr int MT = T / 64, NT = T / 64;  // 32 x 32 tiles per wave
     constexpr int kThreads = 256 * KW, KS = BK / 16 / KW;  // k steps of a wave per stage
     constexpr int TM = T, TN = T, kBuf = kPlanes * T * BK / 8;  // uint4 per operand and buffer
     __shared__ uint4 lds[4 * kBuf];  // [buffer][A, B]
+    __shared__ int votes[2][4 * KW];
     const int lane = threadIdx.x & 63, w = wave_id(), n = lane & 31, hh = lane >> 5;
     const int wm = w & 1, wn = w >> 1 & 1, wk = w >> 2;
 
@@ -186,8 +187,8 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
     Loader<T, BK, kThreads, !TA> ldr_a;
     Loader<T, BK, kThreads, TB> ldr_b;
     constexpr int E = decltype(ldr_a)::E;
-    ldr_a.init(f.A, f.lda, m0, a.g.M);
-    ldr_b.init(f.B, f.ldb, n0, a.g.N);
+    ldr_a.init(threadIdx.x, f.A, f.lda, m0, a.g.M);
+    ldr_b.init(threadIdx.x, f.B, f.ldb, n0, a.g.N);
     // Stages [s0, sf) are whole and go by vector loads.
     const int sf = ldr_a.fast && ldr_b.fast && f.alpha == 1.f ? max(s0, min(s1, (int)(f.K / BK))) : s0;
     f32x16 acc[NT][MT];
@@ -274,58 +275,152 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
     // Sums of few terms are all here (see the top).  Half hh of a wave takes
     // values 4 hh .. 4 hh + 3 of each eight k, and the KW groups of waves take
     // the eights in turn.
+    // What these stages and the results' addresses need is formed again here
+    // (tid is opaque): kept through the loop above it costs the third workgroup
+    // of a CU its registers.
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int n2 = tid & 31, hh2 = tid >> 5 & 1;
+    Loader<T, BK, kThreads, !TA> any_a;
+    Loader<T, BK, kThreads, TB> any_b;
+    any_a.place(tid), any_b.place(tid);
     constexpr int kRow = BK + 4;  // floats from one row to the next
     float* fa = reinterpret_cast<float*>(lds);
     float* fb = fa + TM * kRow;
     static_assert((TM + TN) * kRow * 4 <= sizeof(lds), "a stage in fp32 fits the buffers");
-    for (int s = sf; s < s1; ++s) {
+    // Whether x holds in any thread of the workgroup (a barrier between the two).
+    auto vote = [&](int i, bool x) {
+        const bool any = __any(x);
+        if (lane == 0) votes[i][w] = any;
+    };
+    auto voted = [&](int i) {
+        int v = 0;
+#pragma unroll
+        for (int q = 0; q < 4 * KW; ++q) v |= votes[i][q];
+        return __builtin_amdgcn_readfirstlane(v) != 0;
+    };
+    auto load_stage = [&](int s, float* u, float* v) {  // any stage
         const bool second = s >= a.n0;
         const int64_t k0 = (int64_t)BK * (second ? s - a.n0 : s), K = second ? h.K : f.K;
-        const float alpha = second ? h.alpha : f.alpha;
-        ldr_a.load_any(second ? h.A : f.A, second ? h.lda : f.lda, second ? h.ta == 0 : !TA, m0, a.g.M, k0, K, xa[0]);
-        ldr_b.load_any(second ? h.B : f.B, second ? h.ldb : f.ldb, second ? h.tb != 0 : TB, n0, a.g.N, k0, K, xb[0]);
+        any_a.load_any(second ? h.A : f.A, second ? h.lda : f.lda, second ? h.ta == 0 : !TA, m0, a.g.M, k0, K, u);
+        any_b.load_any(second ? h.B : f.B, second ? h.ldb : f.ldb, second ? h.tb != 0 : TB, n0, a.g.N, k0, K, v);
+        return (int)min<int64_t>(BK, K - k0 + 7) / 8;  // eights of k that hold values
+    };
+    auto fp32_stages = [&](int from) {
+        for (int s = from; s < s1; ++s) {
+            const int eights = load_stage(s, xa[0], xb[0]);
+            const float alpha = s >= a.n0 ? h.alpha : f.alpha;
 #pragma unroll
-        for (int e = 0; e < E; ++e) xa[0][e] *= alpha;
-        lds_barrier();
-        ldr_a.store_f32(fa, kRow, xa[0]);
-        ldr_b.store_f32(fb, kRow, xb[0]);
-        lds_barrier();
-        const int eights = (int)min<int64_t>(BK, K - k0 + 7) / 8;
-        for (int i = wk; i < eights; i += KW) {
-            f32x4 va[MT], vb[NT];
+            for (int e = 0; e < E; ++e) xa[0][e] *= alpha;
+            lds_barrier();
+            any_a.store_f32(fa, kRow, xa[0]);
+            any_b.store_f32(fb, kRow, xb[0]);
+            lds_barrier();
+            for (int i = wk; i < eights; i += KW) {
+                f32x4 va[MT], vb[NT];
 #pragma unroll
-            for (int k = 0; k < MT; ++k)
-                va[k] = *reinterpret_cast<const f32x4*>(fa + (wm * (TM / 2) + 32 * k + n) * kRow + 8 * i + 4 * hh);
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-                vb[j] = *reinterpret_cast<const f32x4*>(fb + (wn * (TN / 2) + 32 * j + n) * kRow + 8 * i + 4 * hh);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
+                for (int k = 0; k < MT; ++k)
+                    va[k] = *reinterpret_cast<const f32x4*>(fa + (wm * (TM / 2) + 32 * k + n2) * kRow + 8 * i + 4 * hh2);
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
+                    vb[j] = *reinterpret_cast<const f32x4*>(fb + (wn * (TN / 2) + 32 * j + n2) * kRow + 8 * i + 4 * hh2);
 #pragma unroll
-                    for (int k = 0; k < MT; ++k) acc[j][k] = mfma_f32(vb[j][e], va[k][e], acc[j][k]);
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+#pragma unroll
+                        for (int k = 0; k < MT; ++k) acc[j][k] = mfma_f32(vb[j][e], va[k][e], acc[j][k]);
+            }
+        }
+    };
+    auto join = [&] {  // the waves' shares of k
+        if constexpr (KW > 1) {
+            static_assert(KW == 2 && MT * NT == 1, "two groups of waves, one 32 x 32 tile each");
+            float* other = reinterpret_cast<float*>(lds) + (w & 3) * 16 * 64 + lane;
+            lds_barrier();
+            if (wk == 1)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) other[64 * r] = acc[0][0][r];
+            lds_barrier();
+            if (wk == 0)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[0][0][r] += other[64 * r];
+        } else {
+            lds_barrier();
+        }
+    };
+    fp32_stages(sf);
+    bool again = false;
+#pragma unroll
+    for (int i = 0; i < 16 * MT * NT; ++i) {
+        const float o = acc[i / (16 * MT)][i / 16 % MT][i % 16];
+        again |= o != o;
+    }
+    vote(0, again);
+    join();
+    if (__builtin_expect(sf > s0 && voted(0), 0)) {
+        // NaN throughout the rows of A and of B that hold one: the other elements count.
+        int* has_nan = reinterpret_cast<int*>(lds) + 16 * 64 * 4;  // [A, B][row], past `other`
+        int here = tid;
+        asm volatile("" : "+v"(here));  // nothing of this is formed ahead
+        for (int i = here; i < TM + TN; i += kThreads) has_nan[i] = 0;
+        lds_barrier();
+        constexpr int kParts = kThreads / (TM + TN);  // threads to a row
+        const int row = here % (TM + TN), part = here / (TM + TN);
+        const bool of_a = row < TM;
+        bool nan = false;
+        for (int t = 0; t < 2; ++t) {
+            const GemmF32Term& x = a.g.terms[t];
+            const int e0 = t == 0 ? min(s0, a.n0) : max(s0, a.n0) - a.n0, e1 = t == 0 ? min(s1, a.n0) : max(s1, a.n0) - a.n0;
+            const int64_t k1 = min((int64_t)BK * e1, x.K);
+            const bool kc = of_a ? x.ta == 0 : x.tb != 0;
+            const int64_t ld = of_a ? x.lda : x.ldb, r = of_a ? min(m0 + row, a.g.M - 1) : min(n0 + row - TM, a.g.N - 1);
+            const float* q = (of_a ? x.A : x.B) + r * (kc ? ld : 1);
+            for (int64_t k = (int64_t)BK * e0 + 8 * part; k < k1; k += 8 * kParts) {
+                if (kc && k + 8 <= k1) {
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        const f32x4_any u = *reinterpret_cast<const f32x4_any*>(q + k + 4 * v);
+                        nan |= u[0] != u[0] || u[1] != u[1] || u[2] != u[2] || u[3] != u[3];
+                    }
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float v = q[min(k + e, k1 - 1) * (kc ? 1 : ld)];
+                        nan |= v != v;
+                    }
+                }
+            }
+        }
+        if (nan) has_nan[row] = 1;
+        lds_barrier();
+        again = false;
+        if (wk == 0)
+#pragma unroll
+            for (int i = 0; i < 16 * MT * NT; ++i) {
+                const int j = i / (16 * MT), k = i / 16 % MT, r = i % 16;
+                const int m = has_nan[wm * (TM / 2) + 32 * k + (here & 31)],
+                          c = has_nan[TM + wn * (TN / 2) + 32 * j + row_of_reg(r, here >> 5 & 1)];
+                again |= (acc[j][k][r] != acc[j][k][r]) & ((m | c) == 0);
+            }
+        vote(1, again);
+        lds_barrier();
+        if (voted(1)) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int k = 0; k < MT; ++k) acc[j][k] = zero16();
+            fp32_stages(s0);
+            join();
         }
     }
+    if (wk != 0) return;
 
-    if constexpr (KW > 1) {
-        static_assert(KW == 2 && MT * NT == 1, "two groups of waves, one 32 x 32 tile each");
-        float* other = reinterpret_cast<float*>(lds) + (w & 3) * 16 * 64 + lane;
-        lds_barrier();
-        if (wk == 1)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) other[64 * r] = acc[0][0][r];
-        lds_barrier();
-        if (wk == 1) return;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[0][0][r] += other[64 * r];
-    }
     float* C = a.whole ? a.g.C : a.g.partial + (int64_t)slice * a.g.M * a.g.N;
     const int64_t ldc = a.whole ? a.g.ldc : a.g.N;
     const float* bias = a.whole ? a.g.bias : nullptr;
     const bool vec = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
-    const int64_t mw = m0 + wm * (TM / 2) + n, nw = n0 + wn * (TN / 2) + 4 * hh;
-    bool nan = false;
+    const int64_t mw = m0 + wm * (TM / 2) + n2, nw = n0 + wn * (TN / 2) + 4 * hh2;
 #pragma unroll
     for (int k = 0; k < MT; ++k) {
         const int64_t m = mw + 32 * k;
@@ -338,10 +433,8 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
                 f32x4 o{acc[j][k][4 * q], acc[j][k][4 * q + 1], acc[j][k][4 * q + 2], acc[j][k][4 * q + 3]};
                 float* d = C + m * ldc + c0;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    nan |= o[e] != o[e];
+                for (int e = 0; e < 4; ++e)
                     if (bias && c0 + e < a.g.N) o[e] += bias[c0 + e];
-                }
                 if (vec && c0 + 4 <= a.g.N) {
                     *reinterpret_cast<f32x4*>(d) = o;
                 } else {
@@ -350,18 +443,6 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_f32_kernel(Args a) {
                         if (c0 + e < a.g.N) d[e] = o[e];
                 }
             }
-    }
-    if (!nan) return;
-    // This lane's elements once more, those that are NaN in plain fp32.
-    for (int i = 0; i < 16 * MT * NT; ++i) {
-        const int64_t m = mw + 32 * (i / (16 * NT)), c = nw + 32 * (i / 16 % NT) + 8 * (i / 4 % 4) + i % 4;
-        if (m >= a.g.M || c >= a.g.N) continue;
-        float* d = C + m * ldc + c;
-        if (*d == *d) continue;
-        const int64_t e0 = min(s0, a.n0), e1 = min(s1, a.n0);
-        float x = exact_dot(a.g.terms[0], m, c, (int64_t)BK * e0, (int64_t)BK * e1, 0.f);
-        x = exact_dot(a.g.terms[1], m, c, (int64_t)BK * (s0 - e0), (int64_t)BK * (s1 - e1), x);
-        *d = x + (bias ? bias[c] : 0.f);
     }
 }
 

@@ -290,3 +290,49 @@ def test_fp32_products_of_one_sign(dev, n, K):
     norm = float((y - ref).norm() / ref.norm()) * 2 ** 24
     print(f"[errs] K {K}: norm {norm:.3f}", flush=True)
     assert norm <= 0.58 * np.sqrt((K + 1) * (2 * K + 1) / (6 * K))
+
+
+@pytest.mark.parametrize("N,I,O,specs", [
+    (2048, 100, 2080, [(5, 2.0, 0, 2080, False, True)]),   # tiles of 128, a rank-r term after six stages and a part
+    (64, 1040, 40, [(3, 2.0, 0, 40, True, False)]),        # k cut into slices, tiles of 64
+    (300, 50, 70, [(40, 1.5, 10, 33, False, False)]),      # an update of its own, added
+])
+@pytest.mark.parametrize("what", ["x inf", "x nan", "W inf", "W nan", "dy inf", "dy nan", "both"])
+def test_fp32_products_keep_inf_and_nan(dev, N, I, O, specs, what):
+    """Infinities and NaN of the operands come out where 64 bits put them, and
+    the elements that they do not reach stay within the K roundings of fp32."""
+    print(f"[case] lora fp32 inf and nan {(N, I, O, specs, what)}", flush=True)
+    rng = np.random.default_rng(N + O)
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    x, W, dy = f(N, I), f(I, O), f(N, O)
+    t, v = ("x", np.inf) if what == "both" else (what.split()[0], np.float32(what.split()[1]))
+    m = dict(x=x, W=W, dy=dy)[t]
+    m[m.shape[0] - 1, m.shape[1] // 3] = v
+    m[m.shape[0] // 2, m.shape[1] // 2] = -v
+    if what == "both":  # an infinity in a row with a NaN, and one that meets another of a column
+        x[N - 1, I // 4] = np.nan
+        W[I // 2, O // 2] = np.inf
+        W[0, O // 2] = -np.inf
+    slices = [dict(A=f(r, I) if at else f(I, r), B=f(c, r) if bt else f(r, c), scale=s, col0=c0,
+                   a_transposed=at, b_transposed=bt) for r, s, c0, c, at, bt in specs]
+    got = _run(dev, x, W, None, slices, False, dy, True)
+    d = lambda a, t: np.asarray(a.T if t else a, np.float64)
+    x6, W6, dy6 = d(x, False), d(W, False), d(dy, False)
+    with np.errstate(invalid="ignore"):
+        y, dx = x6 @ W6, dy6 @ W6.T
+        y_mag, dx_mag = np.abs(x6) @ np.abs(W6), np.abs(dy6) @ np.abs(W6.T)
+        for s in slices:
+            A6, B6, c = d(s["A"], s["a_transposed"]), d(s["B"], s["b_transposed"]), s["col0"]
+            part = slice(c, c + B6.shape[1])
+            y[:, part] += s["scale"] * ((x6 @ A6) @ B6)
+            y_mag[:, part] += s["scale"] * ((np.abs(x6) @ np.abs(A6)) @ np.abs(B6))
+            dx += s["scale"] * ((dy6[:, part] @ B6.T) @ A6.T)
+            dx_mag += s["scale"] * ((np.abs(dy6[:, part]) @ np.abs(B6.T)) @ np.abs(A6.T))
+    for name, g, ref, mag, K in (("y", got["y"], y, y_mag, I), ("dx", got["dx"], dx, dx_mag, O)):
+        g = g.astype(np.float64)
+        print(f"[errs] {name}: {np.isnan(ref).sum()} NaN, {np.isinf(ref).sum()} infinite", flush=True)
+        assert np.array_equal(np.isnan(g), np.isnan(ref)), name
+        assert np.array_equal(g[np.isinf(ref)], ref[np.isinf(ref)]), name
+        ok = np.isfinite(ref)
+        update = 2 + sum(2 * r + 2 for r, *_ in specs)
+        assert (np.abs(g[ok] - ref[ok]) <= (K + update) * 2.0 ** -24 * mag[ok]).all(), name
