@@ -26,7 +26,12 @@
 // where fp32 arithmetic may give inf.  A tile with a NaN that no NaN operand of
 // its row or column explains is computed again, whole, by the fp32 MFMAs; a NaN
 // operand costs its tiles one more pass over their operands (the LM head and
-// loss at 512 x 768 x 20001 with one NaN 0.75 ms, without 0.46).
+// loss at 512 x 768 x 20001 with one NaN 0.75 ms, without 0.46).  So are tiles
+// with a result past the largest float (a1 may be above a), and with one under
+// 2^-80: the third part of an operand under 2^-110 lies below the smallest bf16
+// subnormal, and up to 2^-134 is lost.  In results from 2^-80 on that is
+// under their own rounding while K max(|a|, |b|) < 2^30; operands under 2^-134
+// in a result that is then 0 stay 0.
 //
 // A workgroup (4 waves) owns a T x T tile of C and a range of BK-deep stages
 // of k (of every term in turn, so that a rank-r update is one or two more
@@ -159,6 +164,18 @@ template <int T, int BK, int NT, bool KC> struct Loader {
             *reinterpret_cast<f32x4*>(lds + row * ld + E * kg + 4 * v) =
                 f32x4{x[4 * v], x[4 * v + 1], x[4 * v + 2], x[4 * v + 3]};
     }
+};
+
+// Results that the split does not vouch for (see the top): not finite, or under
+// 2^-80 and not 0.  Twice the bits less one orders zeros above all others.
+struct Doubt {
+    uint32_t least = ~0u;
+    float sum = 0.f;  // NaN once a value is not finite
+    __device__ __forceinline__ void look(float x) {
+        least = min(least, (__float_as_uint(x) << 1) - 1u);
+        sum = fmaf(x, 0.f, sum);
+    }
+    __device__ __forceinline__ bool any() const { return least < ((127u - 80u) << 24) - 1u || sum != sum; }
 };
 
 // TA / TB: term 0's storage.  KW groups of 2 x 2 waves share a stage's 16-deep
@@ -350,13 +367,10 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
         }
     };
     fp32_stages(sf);
-    bool again = false;
+    Doubt doubt;
 #pragma unroll
-    for (int i = 0; i < 16 * MT * NT; ++i) {
-        const float o = acc[i / (16 * MT)][i / 16 % MT][i % 16];
-        again |= o != o;
-    }
-    vote(0, again);
+    for (int i = 0; i < 16 * MT * NT; ++i) doubt.look(acc[i / (16 * MT)][i / 16 % MT][i % 16]);
+    vote(0, doubt.any());
     join();
     if (__builtin_expect(sf > s0 && voted(0), 0)) {
         // NaN throughout the rows of A and of B that hold one: the other elements count.
@@ -376,32 +390,41 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
             const bool kc = of_a ? x.ta == 0 : x.tb != 0;
             const int64_t ld = of_a ? x.lda : x.ldb, r = of_a ? min(m0 + row, a.g.M - 1) : min(n0 + row - TM, a.g.N - 1);
             const float* q = (of_a ? x.A : x.B) + r * (kc ? ld : 1);
-            for (int64_t k = (int64_t)BK * e0 + 8 * part; k < k1; k += 8 * kParts) {
-                if (kc && k + 8 <= k1) {
+            const int64_t step = kc ? 1 : ld;
+            constexpr int U = 8;  // loads in flight
+            int64_t k = (int64_t)BK * e0 + U * part;
+            for (; k + U <= k1; k += U * kParts) {
+                float v[U];
+                if (kc) {
 #pragma unroll
-                    for (int v = 0; v < 2; ++v) {
-                        const f32x4_any u = *reinterpret_cast<const f32x4_any*>(q + k + 4 * v);
-                        nan |= u[0] != u[0] || u[1] != u[1] || u[2] != u[2] || u[3] != u[3];
+                    for (int i = 0; i < U / 4; ++i) {
+                        const f32x4_any u = *reinterpret_cast<const f32x4_any*>(q + k + 4 * i);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[4 * i + e] = u[e];
                     }
                 } else {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const float v = q[min(k + e, k1 - 1) * (kc ? 1 : ld)];
-                        nan |= v != v;
-                    }
+                    for (int e = 0; e < U; ++e) v[e] = q[(k + e) * step];
                 }
+#pragma unroll
+                for (int e = 0; e < U; ++e) nan |= v[e] != v[e];
             }
+            for (const int64_t last = min(k + U, k1); k < last; ++k) nan |= q[k * step] != q[k * step];
         }
         if (nan) has_nan[row] = 1;
         lds_barrier();
-        again = false;
+        bool again = false;
         if (wk == 0)
 #pragma unroll
             for (int i = 0; i < 16 * MT * NT; ++i) {
                 const int j = i / (16 * MT), k = i / 16 % MT, r = i % 16;
                 const int m = has_nan[wm * (TM / 2) + 32 * k + (here & 31)],
                           c = has_nan[TM + wn * (TN / 2) + 32 * j + row_of_reg(r, here >> 5 & 1)];
-                again |= (acc[j][k][r] != acc[j][k][r]) & ((m | c) == 0);
+                float x = acc[j][k][r];
+                asm volatile("" : "+v"(x));  // looked at anew: kept from above it costs a register each
+                Doubt one;
+                one.look(x);
+                again |= one.any() & ((m | c) == 0);
             }
         vote(1, again);
         lds_barrier();

@@ -336,3 +336,26 @@ def test_fp32_products_keep_inf_and_nan(dev, N, I, O, specs, what):
         ok = np.isfinite(ref)
         update = 2 + sum(2 * r + 2 for r, *_ in specs)
         assert (np.abs(g[ok] - ref[ok]) <= (K + update) * 2.0 ** -24 * mag[ok]).all(), name
+
+
+@pytest.mark.parametrize("K", [16, 100, 1040])
+@pytest.mark.parametrize("ex,ey", [(-108, 0), (-112, 20), (-118, 0), (-126, 10), (-130, 40), (-40, -60), (120, -3), (64, 63)])
+def test_fp32_products_over_the_exponents(dev, K, ex, ey):
+    """x of about 2^ex times W of about 2^ey: sums of subnormal and of nearly
+    infinite values are as close to 64 bits as others, K roundings of normal
+    numbers (2^-149 each below those)."""
+    print(f"[case] lora fp32 exponents {(K, ex, ey)}", flush=True)
+    rng = np.random.default_rng(K)
+    f = lambda e, *s: np.ldexp(rng.uniform(-1.0, 1.0, s), e).astype(np.float32)
+    x, W, dy = f(ex, 130, K), f(ey, K, 300), np.zeros((130, 300), np.float32)
+    if ex + ey > 100:
+        x[0], W[:, 0] = np.float32(2.0 ** ex), np.float32(2.0 ** (127 - ex) / K)  # K products that add up to 2^127
+        x[1], W[:, 1] = 3.4e38, np.where(np.arange(K) == 3, 1.0, 0.0)             # one of the largest floats
+    y = _run(dev, x, W, None, [], False, dy)["y"].astype(np.float64)
+    a, b = x.astype(np.float64), W.astype(np.float64)
+    ref, mag = a @ b, np.abs(a) @ np.abs(b)
+    ok = mag < 2.0 ** 127
+    ok[:2, :2] |= np.abs(ref[:2, :2]) <= 3.4e38
+    print(f"[errs] {(np.abs(y - ref)[ok] / mag[ok]).max() * 2 ** 24:.3f} x 2^-24, {ok.sum()} of {ok.size}", flush=True)
+    assert ok.sum() > 3
+    assert (np.abs(y - ref)[ok] <= K * np.maximum(2.0 ** -24 * mag[ok], 2.0 ** -149)).all()
