@@ -62,7 +62,7 @@ struct Args {
     GemmF32 g;
     int tiles_m, tiles_n, slices, stages, per_slice;  // stages of all terms, and of one slice
     int n0;     // stages of term 0
-    int whole;  // one slice and nothing to add to: written to C directly, else to partial
+    int whole;  // one slice: written (or added) to C directly, else to partial
 };
 
 // E values as three planes of packed bf16.
@@ -444,6 +444,27 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
     const float* bias = a.whole ? a.g.bias : nullptr;
     const bool vec = ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
     const int64_t mw = m0 + wm * (TM / 2) + n2, nw = n0 + wn * (TN / 2) + 4 * hh2;
+    if (a.whole && a.g.add) {  // all of C's loads ahead of the stores
+#pragma unroll
+        for (int k = 0; k < MT; ++k) {
+            const float* row = C + min(mw + 32 * k, a.g.M - 1) * ldc;
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t c0 = nw + 32 * j + 8 * q;
+                    f32x4 o;
+                    if (vec && a.g.N % 4 == 0) {
+                        o = *reinterpret_cast<const f32x4*>(row + min(c0, a.g.N - 4));
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[e] = row[min(c0 + e, a.g.N - 1)];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[j][k][4 * q + e] += o[e];
+                }
+        }
+    }
 #pragma unroll
     for (int k = 0; k < MT; ++k) {
         const int64_t m = mw + 32 * k;
@@ -512,7 +533,7 @@ Plan plan(const GemmF32& g) {
     const int slices = cut(tiles(t));
     p.a.per_slice = (stages + slices - 1) / slices;
     p.a.slices = (stages + p.a.per_slice - 1) / p.a.per_slice;
-    p.a.whole = p.a.slices == 1 && !g.add;
+    p.a.whole = p.a.slices == 1;
     return p;
 }
 

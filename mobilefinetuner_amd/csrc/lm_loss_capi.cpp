@@ -75,9 +75,6 @@ size_t chunk_gemms_workspace(const mft_lm_loss_desc* d, int64_t chunk) {
     for (const int64_t nc : {chunk, d->V % chunk ? d->V % chunk : chunk}) {
         const ChunkGemms c = chunk_gemms(d, nc, chunk_ld(chunk));
         for (const mft::GemmF32* g : {&c.z, &c.dh, &c.dw}) w = std::max(w, mft::gemm_f32_workspace(*g));
-        mft::GemmF32 first = c.dh;  // the first chunk's is not added to anything
-        first.add = 0;
-        w = std::max(w, mft::gemm_f32_workspace(first));
     }
     return w;
 }

@@ -268,3 +268,15 @@ def test_lora_validation(capi):
     # backward adds the per-row-chunk partials of grad_A / grad_B ([chunks, max(in, cols), r] fp32;
     # 16-row chunks here: 5 x 256 column waves)
     assert b == 4096 * 1024 * 2 + 4096 * 16 * 4 + 4096 // 16 * 1152 * 16 * 4 + pack + (32 << 20)
+
+
+def test_lora_fp32_updates_need_no_partial_products(capi):
+    """An update that one workgroup per tile sums is added to y (and dx) where
+    it is formed: the workspace of a fused q/k/v projection with three slices
+    holds x . A or g, the k-major copy of an adapter and the gradients'
+    partial sums, and no [N, cols] product."""
+    s = [dict(A=16, B=16, scale=2.0, rank=8, col0=c, cols=768) for c in (0, 768, 1536)]
+    f, b = capi.lora_workspace_size(capi.lora_desc(4096, 768, 2304, capi.MFT_F32, slices=s, grads_for_column_slices=True))
+    u, pack = 4096 * 24 * 4, 768 * 8 * 4
+    assert f == u + pack + 256
+    assert b - f <= 4096 // 16 * 768 * 8 * 4
