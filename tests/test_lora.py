@@ -359,3 +359,31 @@ def test_fp32_products_over_the_exponents(dev, K, ex, ey):
     print(f"[errs] {(np.abs(y - ref)[ok] / mag[ok]).max() * 2 ** 24:.3f} x 2^-24, {ok.sum()} of {ok.size}", flush=True)
     assert ok.sum() > 3
     assert (np.abs(y - ref)[ok] <= K * np.maximum(2.0 ** -24 * mag[ok], 2.0 ** -149)).all()
+
+
+def test_fp32_rows_of_odd_length_cost_no_more(dev):
+    """Rows of 1151 and 1153 floats, every alignment among them, take the same
+    loads as rows of 1152: within 1.6 times their time (1.08 measured; stages
+    of single loads took 2.0)."""
+    import time
+
+    import torch
+    from mobilefinetuner_amd.lora import LoRALinear
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+
+    def ms(I, O):
+        x, W = torch.randn(4096, I, device=dev, generator=g), 0.03 * torch.randn(O, I, device=dev, generator=g)
+        layer, times = LoRALinear(W), []
+        for _ in range(5):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(10):
+                layer.forward(x)
+            torch.cuda.synchronize()
+            times.append(100 * (time.perf_counter() - t))
+        return min(times)
+
+    even, odd = ms(1152, 1152), ms(1151, 1153)
+    print(f"[time] 1152 -> 1152 {even:.4f} ms, 1151 -> 1153 {odd:.4f} ms", flush=True)
+    assert odd <= 1.6 * even
