@@ -510,20 +510,29 @@ struct Plan {
     Args a;
 };
 
-// 128 x 128 tiles where they fill the GPU, with k cut into slices or
-// not; else 64 x 64.  k is cut into slices of at least kMinSlice values until
-// about two workgroups per CU run, where the tiles alone leave more than half
-// of the GPU idle (each slice costs an fp32 tile written and read again).
-constexpr int kMinSlice = 256;
+// 128 x 128 tiles where they fill the GPU, with k cut into slices or not; else
+// 64 x 64.  k is cut into slices of at least kMinSlice values until about two
+// workgroups per CU run, where the tiles alone leave more than half of the GPU
+// idle (each slice costs an fp32 tile written and read again), and of at
+// least kFewSlice until one per CU does (33 x 768 x 768 10.8 -> 9.7 us, 64 x 768
+// x 500 12.9 -> 9.7).  Where 128 x 128 tiles would need slices, a K up to
+// kUncut is shorter in 64 x 64 tiles without (1024 x 1024 x 1024 29 -> 22 us,
+// 2048 x 768 x 768 35 -> 24; at 2048 x 640 x 2048 52 against 44).
+constexpr int kMinSlice = 256, kFewSlice = 96, kUncut = 1536;
 Plan plan(const GemmF32& g) {
     Plan p{};
     const int cus = device_cus();
     auto tiles = [&](int t) { return ((g.M + t - 1) / t) * ((g.N + t - 1) / t); };
     const int64_t K = g.terms[0].K + g.terms[1].K;
     auto cut = [&](int64_t t) {
-        return 2 * t >= cus ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / t, K / kMinSlice));
+        return 2 * t >= cus ? 1
+                            : (int)std::max<int64_t>({1, std::min<int64_t>(2 * cus / t, K / kMinSlice),
+                                                      std::min<int64_t>(cus / t, K / kFewSlice)});
     };
-    p.small = tiles(128) * cut(tiles(128)) < cus;
+    const int64_t t128 = tiles(128);
+    const bool cut128 = 2 * t128 < cus;
+    const int64_t c128 = cut128 ? std::max<int64_t>(1, std::min<int64_t>(2 * cus / t128, K / kMinSlice)) : 1;
+    p.small = t128 * c128 < cus || (cut128 && K <= kUncut);
     const int t = p.small ? 64 : 128, bk = p.small ? 32 : 16;
     p.a.g = g;
     p.a.tiles_m = (int)((g.M + t - 1) / t);
