@@ -49,6 +49,19 @@ hipError_t launch_lora_rowdot(const LoraRowDot& a, hipStream_t st);
 hipError_t launch_lora_pack_kmajor(const float* P, int64_t pk, int64_t pj, int64_t K, int r, float* dst,
                                    hipStream_t st);
 
+// C[n, o] += alpha * sum_k U[n, k] B(k, o) for n < rows, o < cols: a slice's
+// update of y or dx by itself.  B is stored [r, cols], or [cols, r] with bt.
+struct LoraUpdate {
+    const float* U;        // [rows, r] with leading dimension ldu
+    int64_t ldu, rows, cols;
+    const float* B;
+    int bt, r;
+    float alpha;
+    float* C;              // leading dimension ldc
+    int64_t ldc;
+};
+hipError_t launch_lora_update(const LoraUpdate& a, hipStream_t st);
+
 constexpr int64_t kLoraMaxGridY = 65535;  // a launch's grid limit in y (and z)
 
 struct LoraColDot {

@@ -387,3 +387,33 @@ def test_fp32_rows_of_odd_length_cost_no_more(dev):
     even, odd = ms(1152, 1152), ms(1151, 1153)
     print(f"[time] 1152 -> 1152 {even:.4f} ms, 1151 -> 1153 {odd:.4f} ms", flush=True)
     assert odd <= 1.6 * even
+
+
+@pytest.mark.parametrize("N", [1, 7, 8, 1024, 1025])
+@pytest.mark.parametrize("ranks", [(1, 3), (4, 8), (9, 16), (17, 5)])
+@pytest.mark.parametrize("t", [False, True])
+def test_fp32_column_updates(dev, N, ranks, t):
+    """Updates over column ranges by themselves, at the edges of their rows,
+    ranks and 256-column blocks, in y and in dx, against 64 bits: a sum of
+    r terms, one scale and one addition beside the product's K roundings."""
+    print(f"[case] lora fp32 column updates {(N, ranks, t)}", flush=True)
+    rng = np.random.default_rng(N + ranks[0])
+    f = lambda *s: rng.standard_normal(s).astype(np.float32)
+    I, O = 259, 300
+    x, W, dy = f(N, I), f(I, O), f(N, O)
+    slices = [dict(A=f(r, I) if t else f(I, r), B=f(c, r) if t else f(r, c), scale=1.5, col0=c0, a_transposed=t,
+                   b_transposed=t) for r, c0, c in ((ranks[0], 3, 257), (ranks[1], 299, 1), (ranks[1], 0, 256))]
+    got = _run(dev, x, W, None, slices, False, dy, True)
+    d = lambda a, t: np.asarray(a.T if t else a, np.float64)
+    x6, W6, dy6 = d(x, False), d(W, False), d(dy, False)
+    y, y_mag, dx, dx_mag = x6 @ W6, np.abs(x6) @ np.abs(W6), dy6 @ W6.T, np.abs(dy6) @ np.abs(W6.T)
+    for s in slices:
+        A6, B6, c = d(s["A"], t), d(s["B"], t), s["col0"]
+        part = slice(c, c + B6.shape[1])
+        y[:, part] += 1.5 * ((x6 @ A6) @ B6)
+        y_mag[:, part] += 1.5 * ((np.abs(x6) @ np.abs(A6)) @ np.abs(B6))
+        dx += 1.5 * ((dy6[:, part] @ B6.T) @ A6.T)
+        dx_mag += 1.5 * ((np.abs(dy6[:, part]) @ np.abs(B6.T)) @ np.abs(A6.T))
+    update = sum(s["A"].size // I + 3 for s in slices)
+    assert (np.abs(got["y"] - y) <= (I + update) * 2.0 ** -24 * y_mag).all()
+    assert (np.abs(got["dx"] - dx) <= (O + update) * 2.0 ** -24 * dx_mag).all()
