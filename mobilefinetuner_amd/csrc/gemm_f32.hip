@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
     constexpr int kThreads = 256 * KW, KS = BK / 16 / KW;  // k steps of a wave per stage
     constexpr int TM = T, TN = T, kBuf = kPlanes * T * BK / 8;  // uint4 per operand and buffer
     __shared__ uint4 lds[4 * kBuf];  // [buffer][A, B]
-    __shared__ int votes[2][4 * KW];
+    __shared__ int votes[2][4 * KW], nan_rows[2 * T];
     const int lane = threadIdx.x & 63, w = wave_id(), n = lane & 31, hh = lane >> 5;
     const int wm = w & 1, wn = w >> 1 & 1, wk = w >> 2;
 
@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
     constexpr int kRow = BK + 4;  // floats from one row to the next
     float* fa = reinterpret_cast<float*>(lds);
     float* fb = fa + TM * kRow;
-    static_assert((TM + TN) * kRow * 4 <= sizeof(lds), "a stage in fp32 fits the buffers");
+    static_assert((TM + TN) * kRow * 4 + (KW - 1) * 4 * 16 * 64 * 4 <= sizeof(lds), "a stage in fp32 and the shares of k fit the buffers");
     // Whether x holds in any thread of the workgroup (a barrier between the two).
     auto vote = [&](int i, bool x) {
         const bool any = __any(x);
@@ -353,8 +353,7 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
     auto join = [&] {  // the waves' shares of k
         if constexpr (KW > 1) {
             static_assert(KW == 2 && MT * NT == 1, "two groups of waves, one 32 x 32 tile each");
-            float* other = reinterpret_cast<float*>(lds) + (w & 3) * 16 * 64 + lane;
-            lds_barrier();
+            float* other = fb + TN * kRow + (w & 3) * 16 * 64 + lane;
             if (wk == 1)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) other[64 * r] = acc[0][0][r];
@@ -374,10 +373,9 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
     join();
     if (__builtin_expect(sf > s0 && voted(0), 0)) {
         // NaN throughout the rows of A and of B that hold one: the other elements count.
-        int* has_nan = reinterpret_cast<int*>(lds) + 16 * 64 * 4;  // [A, B][row], past `other`
         int here = tid;
         asm volatile("" : "+v"(here));  // nothing of this is formed ahead
-        for (int i = here; i < TM + TN; i += kThreads) has_nan[i] = 0;
+        for (int i = here; i < TM + TN; i += kThreads) nan_rows[i] = 0;
         lds_barrier();
         constexpr int kParts = kThreads / (TM + TN);  // threads to a row
         const int row = here % (TM + TN), part = here / (TM + TN);
@@ -411,15 +409,15 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
             }
             for (const int64_t last = min(k + U, k1); k < last; ++k) nan |= q[k * step] != q[k * step];
         }
-        if (nan) has_nan[row] = 1;
+        if (nan) nan_rows[row] = 1;
         lds_barrier();
         bool again = false;
         if (wk == 0)
 #pragma unroll
             for (int i = 0; i < 16 * MT * NT; ++i) {
                 const int j = i / (16 * MT), k = i / 16 % MT, r = i % 16;
-                const int m = has_nan[wm * (TM / 2) + 32 * k + (here & 31)],
-                          c = has_nan[TM + wn * (TN / 2) + 32 * j + row_of_reg(r, here >> 5 & 1)];
+                const int m = nan_rows[wm * (TM / 2) + 32 * k + (here & 31)],
+                          c = nan_rows[TM + wn * (TN / 2) + 32 * j + row_of_reg(r, here >> 5 & 1)];
                 float x = acc[j][k][r];
                 asm volatile("" : "+v"(x));  // looked at anew: kept from above it costs a register each
                 Doubt one;
