@@ -52,8 +52,8 @@ typedef struct {
     int32_t dtype;         /* element type of logits (dense) or hidden and weight         */
     int32_t ignore_index;  /* skipped label value (reference default -100)                */
     int32_t reduction;     /* mft_reduction; streaming takes MEAN or SUM                  */
-    int32_t chunk;         /* streaming: vocabulary rows per GEMM chunk (0 = 16384, or in
-                              fp32 as many as keep the chunk's logits within 128 MiB)     */
+    int32_t chunk;         /* streaming: vocabulary rows per GEMM chunk (0 = 16384, or more
+                              in fp32 while the workspace stays about that of 16384)      */
 } mft_lm_loss_desc;
 
 /* Workspace bytes of the forward and backward (dense or streaming per desc->H). */

@@ -29,11 +29,14 @@ namespace {
 using namespace mft::capi;
 
 constexpr int64_t kDefaultChunk = 16384;
-// fp32: the default chunk grows while a chunk's logits stay within 128 MiB
-// (half of the last-level cache), so that few positions do not run GEMMs too
-// short to fill the GPU: forward and backward at 512 positions, a vocabulary of
-// 50257 and H 768 take 966 us as one chunk and 1060 as four.
-constexpr int64_t kDefaultLogits = int64_t(1) << 25;
+// fp32: the default chunk grows, so that few positions do not run GEMMs too
+// short to fill the GPU (forward and backward at 512 positions, a vocabulary of
+// 50257 and H 768 take 966 us as one chunk and 1060 as four), while its logits
+// stay within kDefaultLogits values (half of the last-level cache) and within
+// the two buffers of the default chunk and kMoreLogits values: G then takes the
+// logits' place, and the workspace stays about that of the default chunk with
+// the library's 64 MB.
+constexpr int64_t kDefaultLogits = int64_t(1) << 25, kMoreLogits = int64_t(10) << 20;
 constexpr size_t kBlasWorkspace = size_t(64) << 20;
 
 size_t up(size_t x) { return (x + 255) & ~size_t(255); }
@@ -44,9 +47,19 @@ struct Layout {
 
 int64_t chunk_of(const mft_lm_loss_desc* d) {
     int64_t c = d->chunk > 0 ? d->chunk : kDefaultChunk;
-    if (d->chunk == 0 && d->dtype == MFT_F32) c = std::max(c, kDefaultLogits / (d->B * d->S));
+    if (d->chunk == 0 && d->dtype == MFT_F32) {
+        const int64_t N = d->B * d->S, most = std::min(kDefaultLogits / N, 2 * kDefaultChunk + kMoreLogits / N);
+        if (most > c) {  // in chunks of one size (multiples of 64)
+            const int64_t n = (d->V + most - 1) / most;
+            c = std::max(c, ((d->V + n - 1) / n + 63) / 64 * 64);
+        }
+    }
     return c < d->V ? c : d->V;
 }
+
+// Whether a chunk's G is written over its logits (value by value, by the
+// thread that read it).
+bool g_over_logits(const mft_lm_loss_desc* d) { return d->dtype == MFT_F32 && chunk_of(d) > kDefaultChunk; }
 
 // Row stride of a chunk's logits and G: a multiple of 8 elements, so that
 // every row takes vector loads and stores (at a vocabulary of 50257 in one
@@ -94,7 +107,10 @@ Layout layout(const mft_lm_loss_desc* d, bool streaming) {
         // the fused kernels need no fp32 logits chunk
         const bool fused = mft::ce_fused_supported(d->H, d->dtype == MFT_BF16);
         l.z = o, o += fused ? 0 : up(N * chunk_ld((int64_t)c) * 4);
-        l.g = o, o += up(N * chunk_ld((int64_t)c) * esz);
+        if (g_over_logits(d))
+            l.g = l.z;
+        else
+            l.g = o, o += up(N * chunk_ld((int64_t)c) * esz);
         l.blas = o, o += d->dtype == MFT_F32 ? up(chunk_gemms_workspace(d, (int64_t)c)) : kBlasWorkspace;
         // fused forward: (max, sum) pairs per position and vocabulary part
         l.part = o, o += up(N * 2 * mft::kCeFusedMaxRanges * sizeof(float2));

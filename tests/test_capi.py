@@ -280,3 +280,13 @@ def test_lora_fp32_updates_need_no_partial_products(capi):
     u, pack = 4096 * 24 * 4, 768 * 8 * 4
     assert f == u + pack + 256
     assert b - f <= 4096 // 16 * 768 * 8 * 4
+
+
+@pytest.mark.parametrize("N,H,V", [(1, 768, 50257), (4, 1152, 65536), (64, 768, 262144), (128, 640, 262144),
+                                   (333, 768, 50257), (512, 768, 50257), (1024, 1152, 65536), (1500, 640, 262144),
+                                   (4096, 768, 50257), (40000, 640, 32768)])
+def test_streaming_fp32_workspace_is_that_of_the_default_chunk(capi, N, H, V):
+    """Chunks past 16384 rows hold one buffer, so that the workspace is at most
+    8 MB above two buffers of 16384 rows and 64 MB, and the rows' own terms."""
+    f, b = capi.lm_ce_workspace_size(capi.lm_loss_desc(1, N, V, H, capi.MFT_F32))
+    assert f == b <= 2 * 4 * N * min(V, 16384) + (72 << 20) + N * (24 + 1024) + 4096
