@@ -49,6 +49,7 @@
 #include "attn_common.h"
 #include "attn_geometry.h"
 #include "attn_kernels.h"
+#include "prologue_kernels.h"
 
 namespace mft {
 namespace {
@@ -64,6 +65,7 @@ struct Args {
     GemmF32 g;
     int tiles_m, tiles_n, slices, stages, per_slice;  // stages of all terms, and of one slice
     int n0;     // stages of term 0
+    FastDiv per_slice_tiles, fewer_tiles;  // division by tiles_m tiles_n and by the smaller of the two
     int whole;  // one slice: written (or added) to C directly, else to partial
 };
 
@@ -193,10 +195,11 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
     // Tiles that share the larger operand's rows run next to each other on one
     // XCD: the smaller tile count fastest, then the other, then the k slices.
     int i = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    const int per = a.tiles_m * a.tiles_n, slice = i / per;
-    i -= slice * per;
+    const int slice = (int)a.per_slice_tiles.div(i);
+    i -= slice * a.tiles_m * a.tiles_n;
     const bool m_fast = a.tiles_m <= a.tiles_n;
-    const int tm = m_fast ? i % a.tiles_m : i / a.tiles_n, tn = m_fast ? i / a.tiles_m : i % a.tiles_n;
+    const int slow = (int)a.fewer_tiles.div(i), fast = i - slow * (m_fast ? a.tiles_m : a.tiles_n);
+    const int tm = m_fast ? fast : slow, tn = m_fast ? slow : fast;
     const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
     const int s0 = slice * a.per_slice, s1 = min(s0 + a.per_slice, a.stages);
 
@@ -268,9 +271,11 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
         ldr_a.store(next, u);
         ldr_b.store(next + kBuf, v);
 #pragma unroll
-        for (int q = 0; q < 6 * MT * NT * KS; ++q) {  // the split between the MFMAs
+        // The split between the MFMAs (3 to 5 tried at T = 128, 4 to 12 at 64,
+        // where loads along the rows add addresses; up to 8 percent apart).
+        for (int q = 0; q < 6 * MT * NT * KS; ++q) {
             __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(SG_VALU, MT * NT > 1 ? 5 : 8, 0);
+            __builtin_amdgcn_sched_group_barrier(SG_VALU, MT * NT > 1 ? 5 : TB ? 6 : 8, 0);
         }
         fetch(s + 3, u, v);
         lds_barrier();
@@ -541,6 +546,8 @@ Plan plan(const GemmF32& g) {
     p.a.per_slice = (stages + slices - 1) / slices;
     p.a.slices = (stages + p.a.per_slice - 1) / p.a.per_slice;
     p.a.whole = p.a.slices == 1;
+    p.a.per_slice_tiles = FastDiv::make((uint32_t)(p.a.tiles_m * p.a.tiles_n));
+    p.a.fewer_tiles = FastDiv::make((uint32_t)std::min(p.a.tiles_m, p.a.tiles_n));
     return p;
 }
 
