@@ -70,8 +70,6 @@ template <typename T, int VEC> struct alignas(VEC * sizeof(T)) Pack {
     T x[VEC];
 };
 
-constexpr int kFwdThreads = 1024;
-
 // Lanes that span a row of D elements, VEC to a lane: a power of two, so that
 // the rows a workgroup holds at once divide its threads.
 __host__ __device__ constexpr int row_lanes(int D, int VEC) {
@@ -89,20 +87,20 @@ __host__ __device__ constexpr int fwd_lanes(int D, int VEC) {
 
 // Forward: O_i = mean of V over T_i for every masked row, all query heads of
 // the kv head.  Bound by the latency of reading [0, len) and the window.
-// Workgroup = (G rows, batch x kv head, a line's columns), G = 1024 /
-// fwd_lanes (128 rows of 64 bf16 columns): group g of fwd_lanes threads sums
+// Workgroup = (G rows, batch x kv head, a line's columns), G = NT /
+// fwd_lanes (128 rows of 64 bf16 columns with 1024 threads): group g of fwd_lanes threads sums
 // every G-th row of T_r0 (r0 the workgroup's first masked row), eight rows'
 // loads in flight, the groups' sums are added through LDS, and group g then
 // owns row r0 + g, whose T differs from T_r0 by one entering and one leaving
 // row per step: a prefix sum over the groups.  All sums in double.  One thread
 // per column walking the rows alone took 245 us at B 3, Hkv 1, S 1000, D 256,
 // window 512 with lengths down to 390; whole rows to a workgroup 16; this 10.
-template <typename T, int VEC>
-__global__ __launch_bounds__(kFwdThreads) void attn_fwd_masked_rows(MaskedArgs a) {
+template <typename T, int VEC, int NT>
+__global__ __launch_bounds__(NT) void attn_fwd_masked_rows(MaskedArgs a) {
     typedef Pack<T, VEC> P;
-    __shared__ double part[VEC][kFwdThreads], seg[kFwdThreads];
+    __shared__ double part[VEC][NT], seg[NT];
     const int S = a.S, D = a.D, tid = threadIdx.x;
-    const int lanes = fwd_lanes(D, VEC), G = kFwdThreads / lanes, g = tid / lanes;
+    const int lanes = fwd_lanes(D, VEC), G = NT / lanes, g = tid / lanes;
     const int d = ((int)blockIdx.z * lanes + tid % lanes) * VEC;
     const int bk = blockIdx.y, b = bk / a.Hkv, hk = bk % a.Hkv;
     const MaskedRows mr = masked_rows(a, b);
@@ -136,7 +134,7 @@ __global__ __launch_bounds__(kFwdThreads) void attn_fwd_masked_rows(MaskedArgs a
     // A column's G values are handled by Q = G / VEC threads, VEC values each:
     // thread (q, element ce, lane cl).
     const int cols = lanes * VEC, q = tid / cols, ce = (tid % cols) / lanes, cl = tid % lanes;
-    const int Q = kFwdThreads / cols;
+    const int Q = NT / cols;
     double* mine = &part[ce][q * VEC * lanes + cl];  // values s * lanes apart
     double sum = 0.0;
 #pragma unroll
@@ -402,21 +400,29 @@ hipError_t launch_fwd_masked_rows(const AttnShape& s, const void* v, void* o, hi
     MaskedArgs a = masked_args(s);
     a.v = v;
     a.o = o;
-    const int vec = row_vec(s), lanes = fwd_lanes(a.D, vec), rows = kFwdThreads / lanes;
+    // Short sequences take 256 threads: in a call without such rows every
+    // workgroup returns at once, and 1024 threads and 72 KB of LDS for each cost
+    // 0.1 to 0.2 us more (B 4, Hq 12, S 128, bf16 forward 8.52 -> 8.36); with
+    // such rows fewer of them share T_r0 (14.0 -> 11.7, at S 500, D 256 34.9 ->
+    // 31.4).  Past 512 rows the sum over T_r0 outweighs that.
+    const int vec = row_vec(s), lanes = fwd_lanes(a.D, vec), nt = s.S <= 512 ? 256 : 1024, rows = nt / lanes;
     const dim3 grid((unsigned)((s.S + rows - 1) / rows), (unsigned)(s.B * s.Hkv),
                     (unsigned)((a.D + lanes * vec - 1) / (lanes * vec)));
-    const dim3 blk(kFwdThreads);
+#define MFT_MASKED_FWD(T, VEC)                                                                          \
+    do {                                                                                                \
+        if (nt == 256)                                                                                  \
+            hipLaunchKernelGGL((attn_fwd_masked_rows<T, VEC, 256>), grid, dim3(256), 0, st, a);         \
+        else                                                                                            \
+            hipLaunchKernelGGL((attn_fwd_masked_rows<T, VEC, 1024>), grid, dim3(1024), 0, st, a);       \
+    } while (0)
     if (s.bf16) {
-        if (vec > 1)
-            hipLaunchKernelGGL((attn_fwd_masked_rows<bf16, 8>), grid, blk, 0, st, a);
-        else
-            hipLaunchKernelGGL((attn_fwd_masked_rows<bf16, 1>), grid, blk, 0, st, a);
+        if (vec > 1) MFT_MASKED_FWD(bf16, 8);
+        else MFT_MASKED_FWD(bf16, 1);
     } else {
-        if (vec > 1)
-            hipLaunchKernelGGL((attn_fwd_masked_rows<float, 4>), grid, blk, 0, st, a);
-        else
-            hipLaunchKernelGGL((attn_fwd_masked_rows<float, 1>), grid, blk, 0, st, a);
+        if (vec > 1) MFT_MASKED_FWD(float, 4);
+        else MFT_MASKED_FWD(float, 1);
     }
+#undef MFT_MASKED_FWD
     return hipGetLastError();
 }
 

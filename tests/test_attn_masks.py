@@ -159,6 +159,8 @@ def test_window_forward_launch_shapes_agree(orc, dev):
     (1, 2, 1, 67, 250, "f32", True, 5, [1]),          # four rows to a workgroup, one left over
     (2, 4, 1, 333, 64, "bf16", True, 40, [50, 0]),    # 128 rows to a workgroup, the last partly filled
     (2, 2, 2, 129, 256, "bf16", False, 0, [0, 3]),    # not causal: every row of a batch takes one mean
+    (1, 2, 1, 512, 64, "f32", True, 70, [130]),       # the longest rows of 256-thread workgroups
+    (2, 2, 1, 513, 64, "bf16", True, 70, [0, 300]),   # the shortest of 1024
 ], ids=_id)
 def test_rows_without_keys_match_oracle(orc, dev, case):
     """Rows that see no key, at the edges of the row groups and vectors that
