@@ -43,7 +43,10 @@ template <typename T> __device__ __forceinline__ float to_f(T x) { return (float
 // Block-wide (max, sum) merge of per-thread online pairs.
 __device__ __forceinline__ void merge_pair(float& m, float& s, float m2, float s2) {
     const float mn = fmaxf(m, m2);
-    if (mn == -INFINITY) return;
+    if (mn == -INFINITY) {
+        s += s2;  // 0, or the NaN of a value
+        return;
+    }
     s = s * __expf(m - mn) + s2 * __expf(m2 - mn);
     m = mn;
 }
@@ -64,13 +67,14 @@ __device__ __forceinline__ void online_add(float& m, float& s, const float* x) {
     float vm = x[0];
 #pragma unroll
     for (int e = 1; e < VEC; ++e) vm = fmaxf(vm, x[e]);
-    if (vm == -INFINITY) return;  // exp(-inf) adds nothing
     if (vm > m) {
         s *= __expf(m - vm);
         m = vm;
     }
+    // While all are -inf the exponentials are 0, but a NaN, which the maximum passes over, counts.
+    const float base = m == -INFINITY ? 0.f : m;
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) s += __expf(x[e] - m);
+    for (int e = 0; e < VEC; ++e) s += __expf(x[e] - base);
 }
 
 // Elements from p to the next VEC-element boundary.
@@ -127,10 +131,13 @@ __global__ __launch_bounds__(NT) void ce_row_stats(CeArgs a, const T* z, int64_t
         float bm = sm[0], bs = ss[0];
         for (int k = 1; k < NT / 64; ++k) merge_pair(bm, bs, sm[k], ss[k]);
         // merge into the row's running pair (sum kept in double)
-        if (first || a.run_m[n] == -INFINITY) {
+        if (first) {
             a.run_m[n] = bm;
             a.run_s[n] = (double)bs;
-        } else if (bm != -INFINITY) {
+        } else if (a.run_m[n] == -INFINITY || bm == -INFINITY) {  // one of the sums is 0 (or NaN)
+            a.run_m[n] = fmaxf(a.run_m[n], bm);
+            a.run_s[n] += (double)bs;
+        } else {
             const float om = a.run_m[n];
             const float mn = fmaxf(om, bm);
             a.run_s[n] = a.run_s[n] * exp((double)om - (double)mn) + (double)bs * exp((double)bm - (double)mn);

@@ -391,3 +391,42 @@ def test_streaming_fp32_with_a_nan_takes_no_longer(dev):
     finite, with_nan = ms(h), ms(bad)
     print(f"[time] finite {finite:.3f} ms, with a NaN {with_nan:.3f} ms", flush=True)
     assert with_nan <= 2.0 * finite
+
+
+@pytest.mark.parametrize("V", [7, 40, 1001, 20000, 20001])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_a_nan_among_masked_logits(dev, V, dtype):
+    """A row whose logits are -inf but for its label and one NaN has a NaN loss
+    wherever the NaN lies, also with nothing but -inf around it; so has a row
+    of -inf and a NaN, and a row of -inf alone has lse -inf."""
+    import torch
+    from mobilefinetuner_amd import lm_loss as L
+    print(f"[case] NaN among -inf {(V, dtype)}", flush=True)
+    where = sorted({0, 1, 3, V // 3, V // 2, V - 2, V - 1})
+    z = torch.full((1, 2 * len(where) + 3, V), float("-inf"), device=dev)
+    y = torch.full((1, z.shape[1]), V // 4, dtype=torch.int32, device=dev)
+    for r, v in enumerate(where):
+        z[0, r, V // 4] = 1.5
+        z[0, r, v] = float("nan")
+        z[0, len(where) + r, v] = float("nan")
+    z[0, 2 * len(where), V // 4] = 1.5
+    _, lse = L.lm_cross_entropy(z.to(torch.bfloat16 if dtype == "bf16" else torch.float32), y, -100, "none")
+    lse = lse[0].cpu()
+    assert torch.isnan(lse[: 2 * len(where)]).all(), lse
+    assert lse[2 * len(where)] == 1.5 and lse[2 * len(where) + 1] == float("-inf")
+
+
+@pytest.mark.parametrize("at", [0, 300, 999])
+def test_streaming_nan_among_masked_rows(dev, at):
+    """The same over chunks of the vocabulary: one of only -inf and a NaN."""
+    import torch
+    from mobilefinetuner_amd import lm_loss as L
+    print(f"[case] streaming NaN among -inf {at}", flush=True)
+    h, w = torch.ones(1, 5, 16, device=dev), torch.full((1000, 16), float("-inf"), device=dev)
+    y = torch.full((1, 5), 600, dtype=torch.int32, device=dev)
+    w[600] = 0.25
+    _, lse = L.streaming_lm_cross_entropy(h, w, y, -100, "sum", 250)
+    assert torch.equal(lse[0, :4].cpu(), torch.full((4,), 4.0))
+    w[at] = float("nan")
+    loss, lse = L.streaming_lm_cross_entropy(h, w, y, -100, "sum", 250)
+    assert torch.isnan(loss).all() and torch.isnan(lse[0, :4]).all()
