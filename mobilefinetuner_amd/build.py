@@ -90,7 +90,7 @@ def build(verbose: bool = True) -> str:
     with cf.ThreadPoolExecutor(workers) as ex:
         objs = list(ex.map(_compile, srcs))
     tmp = LIB + ".tmp"
-    # rocBLAS runs the plain GEMMs of the streaming LM cross-entropy.
+    # rocBLAS runs the plain bf16 GEMMs of the streaming LM cross-entropy and of the LoRA layer.
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs, "-L/opt/rocm/lib", "-lrocblas",
            "-Wl,-rpath,/opt/rocm/lib"]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -16,12 +16,17 @@
 // of the error against 64 bits in 2^-24 of the result, normal operands, beside
 // fp32 MFMAs throughout: K 16 1.0 (1.2), 100 1.7 (3.0), 768 2.9 (8.3); of one
 // sign, 2048 rows: K 768 4.9 (7.1), 4096 9.9 (15.9).
+// (Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial intelligence
+// datatype for higher-precision computations", ARITH 2019, split fp32 so.)
 // What it gives (us, TFLOP/s of the fp32 product; rocBLAS's fp32 kernels beside
-// it): 512 x 16384 x 768 70 us, 183 (96 us); 512 x 768 x 16384 80 us, 161 (124
-// us, 880 without its split-k kernels); 2048 x 16384 x 1024 339 us, 203 (482
-// us), 1.2 PFLOP/s of bf16 products; 509 x 768 x 2304 23 us (21 us).  Bound by the
-// barrier per stage and the LDS traffic (72 KB per 128 x 128 x 16 stage)
-// beside the MFMAs.
+// it, one box): 512 x 16384 x 768 73 us, 176 (102 us); 512 x 768 x 16384 86 us,
+// 150 (895 us); 2048 x 16384 x 1024 351 us, 196 (458 us); 509 x 2304 x 768 25 us
+// (27 us), 509 x 768 x 2304 24 us (20 us).  At T = 128 (512 x 50257 x 768 and its
+// two gradients) the matrix units are busy 48 to 55 percent of the cycles, at
+// the 1.8 to 2 GHz that the card holds under them, the VALU, which splits, 39,
+// half of that beside them, and the LDS 28 to 37; half of the waves' cycles wait
+// for issue.  At T = 64 the serial chain of a stage bounds it (matrix units 14 to
+// 18 percent).
 // Infinities: a remainder of inf, or 0 * inf among the six products, is NaN
 // where fp32 arithmetic may give inf.  A tile with a NaN that no NaN operand of
 // its row or column explains is computed again, whole, by the fp32 MFMAs; a NaN

@@ -3,7 +3,8 @@
 // The layer is GEMMs plus element-wise staging.  Row-major throughout, R =
 // sum of the slices' ranks, s_i = scale_i:
 //   (fp32 W: y and dx are one product each on the bf16 matrix units, the
-//    update of one slice and the bias with it; gemm_f32.h)
+//    update of one slice and the bias with it, gemm_f32.h; other slices'
+//    updates are added by lora_update or, from some rank on, gemm_f32)
 //   forward   y  = x . W (+ bias)                 rocBLAS; bf16 W: x staged
 //                                                  to bf16 by the first rowdot
 //                                                  (bf16 W [out, in] with one

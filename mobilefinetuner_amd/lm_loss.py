@@ -1,7 +1,7 @@
 """torch-tensor plumbing over the LM cross-entropy C ABI (include/mft/lm_loss.h).
 
-The arithmetic is in libmft_attn.so (HIP kernels, rocBLAS for the streaming
-variant's chunk GEMMs).  These helpers allocate outputs and workspace as torch
+The arithmetic is in libmft_attn.so (HIP kernels; rocBLAS for the bf16
+streaming variant's gradient GEMMs, and its logits where H % 64).  These helpers allocate outputs and workspace as torch
 tensors on the current device and enqueue on torch's current stream; there is
 no CPU path.  Semantics are ops::lm_cross_entropy /
 ops::streaming_lm_cross_entropy (core/lm_loss.h): labels[b, s + 1] scores
