@@ -440,7 +440,10 @@ __global__ __launch_bounds__(256 * KW, 3) void gemm_f32_kernel(Args a) {
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int k = 0; k < MT; ++k) acc[j][k] = zero16();
+                for (int k = 0; k < MT; ++k) {
+                    acc[j][k] = zero16();
+                    asm volatile("" : "+v"(acc[j][k]));  // as above
+                }
             fp32_stages(s0);
             join();
         }

@@ -313,7 +313,7 @@ def test_dense_unaligned_rows(dev, case):
 ], ids=lambda c: "B{}S{}H{}V{}-c{}".format(*c))
 def test_streaming_fp32_products(dev, case):
     """The fp32 products at the edges of their tiles and k stages, against
-    double precision.  Six bf16 products stand for one fp32 product to 2^-21
+    double precision.  Six bf16 products stand for one fp32 product to 2^-23.9
     at worst and the sums are fp32: 4e-6 of the norm (a plain fp32 product of
     the largest of these has 2e-6), 1e-5 for the loss and lse."""
     import torch
