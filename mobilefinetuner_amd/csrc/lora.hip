@@ -1,4 +1,4 @@
-// Element-wise kernels of the LoRA linear layer (C ABI in include/mft/lora.h,
+// Element-wise and rank-r kernels of the LoRA linear layer (C ABI in include/mft/lora.h,
 // GEMMs in lora_capi.cpp).
 //
 //   lora_round_bf16   fp32 -> bf16 operand staging for the bf16 MFMA GEMMs;
@@ -9,6 +9,8 @@
 //                     per element a rank-long double dot product, then one
 //                     fp32 multiply and add, element for element as the
 //                     reference rounds them (fp contract off).
+//   lora_rowdot, lora_coldot   u, g and the adapters' gradients; each below.
+//   lora_update       a slice's low-rank update of y or dx by itself.
 #include <hip/hip_runtime.h>
 
 #include "lora_kernels.h"
